@@ -29,13 +29,21 @@
 //              (nibbles j and j+4 of a word decode together).  Rows M .. roundup(M, 32) - 1
 // are written as zeros, so the GEMM reads whole fragments.
 //
-// Mapping: one wave per row; lane l takes the 8-element output slots l, l+64,
-// ... (slot 8c + 2t + h: chunk c, step t, half h).  K <= 4096 and M >= 1024:
-// eight rows per 512-thread workgroup, whose slots meet in LDS and leave as
-// whole 128-byte lines of the fragments.  Otherwise four rows per 256-thread
-// workgroup, each lane storing its own 16-byte slots; rows with K <= 12288
-// keep their values in registers between the max pass and the conversion
-// pass, longer rows reload them (cache hits), four slots in flight per lane.
+// Mapping: a row is shared by WPR waves, each lane taking up to NR output slots
+// of 8 elements (slot 8c + 2t + h: chunk c, step t, half h) that it holds in
+// registers between the max pass and the conversion; the waves' maxima meet in
+// LDS.  Bound: HBM / L2 traffic for many rows, one memory round trip for few, so
+// what counts is loads in flight: WPR grows until the launch has 16 waves per CU
+// or a lane one slot (below).  With one wave per row, which reread rows longer
+// than 12288, 45 f32 rows of 12288 took 18.2 us, now 5.3; 512 bf16 rows of 12288
+// 27.8 -> 11.7; 2048 f32 rows of 12288 113 -> 29.6 us (5.1 TB/s of reads and
+// writes); 45 rows of 4096 6.6 -> 4.8.
+// From kXprepWholeMinRows rows (there are enough of them), and from
+// kXprepPartsMinRows when K >= kXprepPartsMinK, eight rows share a workgroup and
+// their slots leave as whole 128-byte lines; otherwise each lane stores its own
+// 16-byte slots, four rows or fewer to a workgroup (512 rows: K = 1024 3.6 us
+// against 3.9 by lines, K = 3072 6.0 against 6.4; K = 4096 6.9 against 6.2,
+// K = 12288 13.3 against 11.7).
 // NaN and inf: the row's scale is taken as 2^15 and the non-finite values
 // propagate to the row's outputs.
 #include "device_common.hpp"
@@ -48,8 +56,6 @@ namespace {
 typedef _Float16 xh2 __attribute__((ext_vector_type(2)));
 typedef float xf2 __attribute__((ext_vector_type(2)));
 typedef float xf4 __attribute__((ext_vector_type(4)));
-
-constexpr int kXprepWaves = 4;
 
 // The 8 activations of output slot `slot` of a row: two runs of 4 k, at
 // k0 and k0 + RUN2 (NIB: 16, BYTE and WORD: 4, i.e. one run of 8).
@@ -104,19 +110,21 @@ __device__ __forceinline__ size_t frag_offset(uint32_t m, uint32_t slot, uint32_
 }
 
 // NIB and BYTE pair (v0, v2), (v1, v3), (v4, v6), (v5, v7); WORD pairs (v0, v4),
-// (v1, v5), (v2, v6), (v3, v7).  Non-temporal stores: the staged operand is
-// read by the next kernel, not by this one, and streaming it out during the
-// kernel rather than leaving dirty L2 lines for the end-of-kernel write-back
-// measured 7.3 -> 6.1 us at M = 2048, K = 1024.
+// (v1, v5), (v2, v6), (v3, v7).
 typedef uint32_t xu4 __attribute__((ext_vector_type(4)));
 template <uint32_t LAYOUT>
 __device__ __forceinline__ xu4 pack8(const float (&v)[8], int sh) {
     return LAYOUT == XFRAG_WORD ? xu4{pk(v[0], v[4], sh), pk(v[1], v[5], sh), pk(v[2], v[6], sh), pk(v[3], v[7], sh)}
                                 : xu4{pk(v[0], v[2], sh), pk(v[1], v[3], sh), pk(v[4], v[6], sh), pk(v[5], v[7], sh)};
 }
+// Plain stores: a slot is an eighth of its 128-byte line, and L2 merges the
+// rows' slots (non-temporal stores of the pieces took 20.1 us against 13.3 for
+// 512 rows of 12288).  Whole lines (xprep_lines_kernel) do leave non-temporally:
+// the next kernel reads them, and streaming them out beats leaving dirty lines
+// for the end of the kernel (7.3 -> 6.1 us at M = 2048, K = 1024).
 template <uint32_t LAYOUT>
 __device__ __forceinline__ void store8(uint16_t* xh, size_t off, const float (&v)[8], int sh) {
-    __builtin_nontemporal_store(pack8<LAYOUT>(v, sh), gptr_mut<xu4>(xh + off));
+    *gptr_mut<xu4>(xh + off) = pack8<LAYOUT>(v, sh);
 }
 
 // Maximum over the wave (unsigned), every lane receiving it.
@@ -129,148 +137,201 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
     return v;
 }
 
-// NR > 0: up to NR slots per lane held in registers (K <= 512·NR); NR = 0: reload.
-template <bool XBF16, uint32_t LAYOUT, int NR>
-__global__ __launch_bounds__(kXprepWaves * 64) void xprep_kernel(const void* __restrict__ x, uint32_t M, uint32_t Mp,
-                                                                  uint32_t K, uint16_t* __restrict__ xh,
-                                                                  float* __restrict__ rs) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t m = blockIdx.x * (uint32_t)kXprepWaves + (threadIdx.x >> 6);
-    if (m >= Mp) return;
-    const uint32_t slots = K / 8u, ksteps = K / 16u;
-    if (m >= M) {  // padding row: zeros
-        const float z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (uint32_t g = lane; g < slots; g += 64u) store8<LAYOUT>(xh, frag_offset(m, g, ksteps), z, 0);
-        if (lane == 0) gptr_mut<float>(rs)[m] = 0.0f;
-        return;
-    }
-    const size_t row = (size_t)m * K;
-    uint32_t mx = 0;
-    float v[NR > 0 ? NR : 1][8];
-    if constexpr (NR > 0) {
-#pragma unroll
-        for (int i = 0; i < NR; i++) {
-            const uint32_t g = lane + 64u * (uint32_t)i;
-            if (g < slots) {
-                load8<XBF16, LAYOUT>(x, row, g, v[i]);
-                mx = absbits_max8(v[i], mx);
-            }
-        }
-    } else {
-        // four slots in flight per lane (cache hits on the second pass)
-        for (uint32_t g0 = lane; g0 < slots; g0 += 256u) {
-            float t[4][8];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (g0 + 64u * i < slots) load8<XBF16, LAYOUT>(x, row, g0 + 64u * i, t[i]);
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (g0 + 64u * i < slots) mx = absbits_max8(t[i], mx);
-        }
-    }
-    mx = wave_umax(mx);
-    // binary exponent e of the largest magnitude (|x| < 2^e): biased exponent
-    // - 126 for normal values; zero and subnormal rows clamp to -110 (so
-    // 2^(15 - e) stays a normal f32); inf / NaN rows take e = 0
-    int e = mx >= 0x7F800000u ? 0 : (int)(mx >> 23) - 126;
-    e = e < -110 ? -110 : e;
-    const int sh = 15 - e;
-    if constexpr (NR > 0) {
-#pragma unroll
-        for (int i = 0; i < NR; i++) {
-            const uint32_t g = lane + 64u * (uint32_t)i;
-            if (g < slots) store8<LAYOUT>(xh, frag_offset(m, g, ksteps), v[i], sh);
-        }
-    } else {
-        for (uint32_t g0 = lane; g0 < slots; g0 += 256u) {
-            float t[4][8];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (g0 + 64u * i < slots) load8<XBF16, LAYOUT>(x, row, g0 + 64u * i, t[i]);
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (g0 + 64u * i < slots) store8<LAYOUT>(xh, frag_offset(m, g0 + 64u * i, ksteps), t[i], sh);
-        }
-    }
-    if (lane == 0) gptr_mut<float>(rs)[m] = ldexpf(1.0f, e - 15);
+// Scale of a row whose largest |x| has the bits mx: binary exponent e of the
+// largest magnitude (|x| < 2^e): biased exponent - 126 for normal values; zero
+// and subnormal rows clamp to -110 (so 2^(15 - e) stays a normal f32); inf /
+// NaN rows take e = 0.
+__device__ __forceinline__ int row_exponent(uint32_t mx) {
+    const int e = mx >= 0x7F800000u ? 0 : (int)(mx >> 23) - 126;
+    return e < -110 ? -110 : e;
 }
 
-// Rows of K <= kXprepLinesMaxK: eight rows per 512-thread workgroup (one wave
-// each), the rows' 16-byte slots gathered in LDS so that the eight rows' slots
-// of one (k step, half), consecutive in the fragment, leave as one 128-byte
-// line: a store instruction writes 8 whole lines instead of 64 pieces of 64
-// lines.
-constexpr uint32_t kXprepLinesRows = 8, kXprepLinesMaxK = 4096, kXprepLinesMinRows = 1024;
-template <bool XBF16, uint32_t LAYOUT, int NR>
-__global__ __launch_bounds__(kXprepLinesRows * 64) void xprep_lines_kernel(const void* __restrict__ x, uint32_t M,
-                                                                          uint32_t K, uint16_t* __restrict__ xh,
-                                                                          float* __restrict__ rs) {
-    static_assert(NR > 0 && NR * 512 <= (int)kXprepLinesMaxK, "the row's slots are held in registers");
-    extern __shared__ xu4 tile[];  // [slot][row of the eight]: K · 16 bytes
-    const uint32_t lane = threadIdx.x & 63u, r = threadIdx.x >> 6;
-    const uint32_t m0 = blockIdx.x * kXprepLinesRows, m = m0 + r;  // Mp is a multiple of 8: m < Mp
+// The maximum of a row's WPR waves (wave wr of row r), every lane receiving it.
+// Every wave of the workgroup calls it.
+template <uint32_t WPR>
+__device__ __forceinline__ uint32_t row_umax(uint32_t v, uint32_t r, uint32_t wr, uint32_t lane, uint32_t* part) {
+    v = wave_umax(v);
+    if constexpr (WPR > 1) {
+        if (lane == 0) part[r * WPR + wr] = v;
+        __syncthreads();
+        v = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < WPR; i++) {
+            const uint32_t u = part[r * WPR + i];
+            v = u > v ? u : v;
+        }
+    }
+    return v;
+}
+
+// Workgroup of R = max(1, 4 / WPR) rows; K <= 512·WPR·NR.
+template <bool XBF16, uint32_t LAYOUT, int NR, uint32_t WPR>
+__global__ __launch_bounds__((WPR > 4u ? WPR : 4u) * 64u) void xprep_kernel(const void* __restrict__ x, uint32_t M,
+                                                                           uint32_t K, uint16_t* __restrict__ xh,
+                                                                           float* __restrict__ rs) {
+    constexpr uint32_t R = WPR > 4u ? 1u : 4u / WPR;
+    __shared__ uint32_t part[R * WPR];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t r = wave / WPR, wr = wave % WPR;
+    const uint32_t m = blockIdx.x * R + r;  // below M rounded up to 32: R divides 32
     const uint32_t slots = K / 8u, ksteps = K / 16u;
-    const bool real = m < M;  // rows M .. Mp - 1 are zeros
+    const bool real = m < M;  // rows M .. roundup(M, 32) - 1 are zeros
     const size_t row = real ? (size_t)m * K : 0u;
     uint32_t mx = 0;
     float v[NR][8];
 #pragma unroll
     for (int i = 0; i < NR; i++) {
-        const uint32_t g = lane + 64u * (uint32_t)i;
+        const uint32_t g = 64u * (wr + WPR * (uint32_t)i) + lane;
+        if (g < slots) load8<XBF16, LAYOUT>(x, row, g, v[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+        const uint32_t g = 64u * (wr + WPR * (uint32_t)i) + lane;
         if (g < slots) {
-            load8<XBF16, LAYOUT>(x, row, g, v[i]);
 #pragma unroll
             for (int q = 0; q < 8; q++) v[i][q] = real ? v[i][q] : 0.0f;
             mx = absbits_max8(v[i], mx);
         }
     }
-    mx = wave_umax(mx);
-    int e = mx >= 0x7F800000u ? 0 : (int)(mx >> 23) - 126;
-    e = e < -110 ? -110 : e;
-    const int sh = 15 - e;
+    const int e = row_exponent(row_umax<WPR>(mx, r, wr, lane, part));
 #pragma unroll
     for (int i = 0; i < NR; i++) {
-        const uint32_t g = lane + 64u * (uint32_t)i;
-        if (g < slots) tile[g * kXprepLinesRows + r] = pack8<LAYOUT>(v[i], sh);
+        const uint32_t g = 64u * (wr + WPR * (uint32_t)i) + lane;
+        if (g < slots) store8<LAYOUT>(xh, frag_offset(m, g, ksteps), v[i], 15 - e);
     }
-    if (lane == 0) gptr_mut<float>(rs)[m] = real ? ldexpf(1.0f, e - 15) : 0.0f;
-    __syncthreads();
-    // piece p = (slot g, row r') of the eight rows: line g at frag_offset(m0, g)
-    for (uint32_t p = threadIdx.x; p < slots * kXprepLinesRows; p += kXprepLinesRows * 64u) {
-        const uint32_t g = p / kXprepLinesRows, rr = p % kXprepLinesRows;
-        __builtin_nontemporal_store(tile[p], gptr_mut<xu4>(xh + frag_offset(m0 + rr, g, ksteps)));
+    if (lane == 0 && wr == 0) gptr_mut<float>(rs)[m] = real ? ldexpf(1.0f, e - 15) : 0.0f;
+}
+
+// Eight rows per workgroup of 8·WPR waves, the rows' 16-byte slots gathered in
+// LDS so that the eight rows' slots of one (k step, half), consecutive in the
+// fragment, leave as one 128-byte line: a store instruction writes 8 whole
+// lines instead of 64 pieces of 64 lines.  Workgroup (., p) converts slots
+// [p·CAP, (p + 1)·CAP) of the rows, CAP = 64·WPR·NR (held in registers), and
+// reads the others for the maximum only, so fewer rows than CUs·8 still fill
+// the chip (PARTS; otherwise one workgroup holds the rows whole).  The LDS tile holds SEG slots per lane, so a long part passes
+// through it in NR / SEG turns.
+constexpr uint32_t kXprepLinesRows = 8, kXprepWholeMinRows = 1024, kXprepPartsMinRows = 256, kXprepPartsMinK = 4096;
+template <bool XBF16, uint32_t LAYOUT, int NR, int SEG, uint32_t WPR, bool PARTS>
+__global__ __launch_bounds__(kXprepLinesRows * WPR * 64) void xprep_lines_kernel(const void* __restrict__ x, uint32_t M,
+                                                                                uint32_t K, uint16_t* __restrict__ xh,
+                                                                                float* __restrict__ rs) {
+    static_assert(NR % SEG == 0, "whole turns");
+    constexpr uint32_t T = kXprepLinesRows * WPR * 64u, kStep = 64u * WPR, kCap = kStep * NR;
+    extern __shared__ xu4 tile[];  // [slot of the turn][row of the eight]
+    __shared__ uint32_t part[kXprepLinesRows * WPR];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t r = wave / WPR, wr = wave % WPR;
+    const uint32_t m0 = blockIdx.x * kXprepLinesRows, m = m0 + r;  // rows rounded up to 32: a multiple of 8
+    const uint32_t slots = K / 8u, ksteps = K / 16u, s0 = PARTS ? blockIdx.y * kCap : 0u;
+    const bool real = m < M;  // rows M .. roundup(M, 32) - 1 are zeros
+    const size_t row = real ? (size_t)m * K : 0u;
+    const uint32_t l0 = 64u * wr + lane;
+    uint32_t mx = 0;
+    float v[NR][8];
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+        const uint32_t g = s0 + l0 + kStep * (uint32_t)i;
+        if (g < slots) load8<XBF16, LAYOUT>(x, row, g, v[i]);
     }
+    for (uint32_t b = 0; PARTS && b < slots; b += kCap) {  // the other workgroups' parts
+        if (b == s0) continue;
+        constexpr int U = NR < 4 ? NR : 4;
+#pragma unroll
+        for (int i0 = 0; i0 < NR; i0 += U) {
+            float o[U][8];
+#pragma unroll
+            for (int i = 0; i < U; i++) {
+                const uint32_t g = b + l0 + kStep * (uint32_t)(i0 + i);
+                load8<XBF16, LAYOUT>(x, row, g < slots ? g : 0u, o[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < U; i++) mx = absbits_max8(o[i], mx);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+        if (s0 + l0 + kStep * (uint32_t)i < slots) mx = absbits_max8(v[i], mx);
+    }
+    const int e = row_exponent(row_umax<WPR>(mx, r, wr, lane, part));
+    if (lane == 0 && wr == 0 && s0 == 0) gptr_mut<float>(rs)[m] = real ? ldexpf(1.0f, e - 15) : 0.0f;
+#pragma unroll
+    for (int s = 0; s < NR / SEG; s++) {
+        const uint32_t t0 = s0 + kStep * (uint32_t)(SEG * s);  // the turn's first slot
+        if (s > 0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < SEG; i++) {
+            const uint32_t g = l0 + kStep * (uint32_t)i;
+            if (t0 + g < slots) {
+                const xu4 h = pack8<LAYOUT>(v[SEG * s + i], 15 - e);
+                tile[g * kXprepLinesRows + r] = real ? h : xu4{0, 0, 0, 0};
+            }
+        }
+        __syncthreads();
+        // piece p = (slot g, row r') of the eight rows: line g at frag_offset(m0, g)
+        const uint32_t n = t0 >= slots ? 0u : (slots - t0 < kStep * SEG ? slots - t0 : kStep * SEG);
+        for (uint32_t p = threadIdx.x; p < n * kXprepLinesRows; p += T) {
+            const uint32_t g = t0 + p / kXprepLinesRows, rr = p % kXprepLinesRows;
+            __builtin_nontemporal_store(tile[p], gptr_mut<xu4>(xh + frag_offset(m0 + rr, g, ksteps)));
+        }
+    }
+}
+
+template <bool XBF16, uint32_t LAYOUT, int NR, uint32_t WPR>
+hipError_t launch_rows(const void* x, uint32_t M, uint32_t Mp, uint32_t K, uint16_t* xh, float* rs, hipStream_t st) {
+    constexpr uint32_t R = WPR > 4u ? 1u : 4u / WPR;
+    hipLaunchKernelGGL((xprep_kernel<XBF16, LAYOUT, NR, WPR>), dim3(Mp / R), dim3(R * WPR * 64u), 0, st, x, M, K, xh, rs);
+    return hipGetLastError();
+}
+template <bool XBF16, uint32_t LAYOUT, uint32_t WPR>
+hipError_t launch_rows(const void* x, uint32_t M, uint32_t Mp, uint32_t K, uint16_t* xh, float* rs, hipStream_t st) {
+    const uint32_t nr = (K / 8u + 64u * WPR - 1u) / (64u * WPR);  // slots per lane
+    if (nr <= 1u) return launch_rows<XBF16, LAYOUT, 1, WPR>(x, M, Mp, K, xh, rs, st);
+    if (nr <= 2u) return launch_rows<XBF16, LAYOUT, 2, WPR>(x, M, Mp, K, xh, rs, st);
+    if (nr <= 4u) return launch_rows<XBF16, LAYOUT, 4, WPR>(x, M, Mp, K, xh, rs, st);
+    if (nr <= 8u) return launch_rows<XBF16, LAYOUT, 8, WPR>(x, M, Mp, K, xh, rs, st);
+    return hipErrorInvalidValue;
+}
+template <bool XBF16, uint32_t LAYOUT, int NR, int SEG, uint32_t WPR, bool PARTS>
+hipError_t launch_lines(const void* x, uint32_t M, uint32_t Mp, uint32_t K, uint16_t* xh, float* rs, hipStream_t st) {
+    constexpr uint32_t cap = 64u * WPR * NR, turn = 64u * WPR * SEG;
+    const uint32_t slots = K / 8u;
+    const size_t lds = (size_t)(slots < turn ? slots : turn) * kXprepLinesRows * 16u;  // 64 KiB at most
+    hipLaunchKernelGGL((xprep_lines_kernel<XBF16, LAYOUT, NR, SEG, WPR, PARTS>),
+                       dim3(Mp / kXprepLinesRows, (slots + cap - 1u) / cap), dim3(kXprepLinesRows * WPR * 64u), lds, st,
+                       x, M, K, xh, rs);
+    return hipGetLastError();
 }
 
 template <bool XBF16, uint32_t LAYOUT>
 hipError_t launch_xprep(const void* x, uint32_t M, uint32_t K, uint16_t* xh, float* rs, hipStream_t st) {
-    const uint32_t Mp = (M + 31u) & ~31u;
-    const dim3 grid((Mp + kXprepWaves - 1) / kXprepWaves), block(kXprepWaves * 64);
-    const uint32_t slots = K / 8u;
-    // (on fewer rows the 8-row workgroups are too few: M = 512, K = 1024 took
-    // 14.5 us per prefill call against 14.1 with 4-row workgroups; at M =
-    // 2048 the whole lines gave 28.0 -> 26.8 us at K = 1024, 38.7 -> 30.5 us
-    // at K = 3072)
-    if (K <= kXprepLinesMaxK && Mp >= kXprepLinesMinRows) {
-        const dim3 lgrid(Mp / kXprepLinesRows), lblock(kXprepLinesRows * 64);
-        const size_t lds = (size_t)K * 16u;  // 64 KiB at most
-        if (slots <= 64u)
-            hipLaunchKernelGGL((xprep_lines_kernel<XBF16, LAYOUT, 1>), lgrid, lblock, lds, st, x, M, K, xh, rs);
-        else if (slots <= 128u)
-            hipLaunchKernelGGL((xprep_lines_kernel<XBF16, LAYOUT, 2>), lgrid, lblock, lds, st, x, M, K, xh, rs);
-        else if (slots <= 256u)
-            hipLaunchKernelGGL((xprep_lines_kernel<XBF16, LAYOUT, 4>), lgrid, lblock, lds, st, x, M, K, xh, rs);
-        else hipLaunchKernelGGL((xprep_lines_kernel<XBF16, LAYOUT, 8>), lgrid, lblock, lds, st, x, M, K, xh, rs);
-        return hipGetLastError();
+    const uint32_t Mp = (M + 31u) & ~31u, slots = K / 8u;
+    if (Mp >= kXprepWholeMinRows && slots <= 1536u) {
+        if (slots <= 64u) return launch_lines<XBF16, LAYOUT, 1, 1, 1, false>(x, M, Mp, K, xh, rs, st);
+        if (slots <= 128u) return launch_lines<XBF16, LAYOUT, 1, 1, 2, false>(x, M, Mp, K, xh, rs, st);
+        if (slots <= 256u) return launch_lines<XBF16, LAYOUT, 2, 2, 2, false>(x, M, Mp, K, xh, rs, st);
+        if (slots <= 512u) return launch_lines<XBF16, LAYOUT, 4, 4, 2, false>(x, M, Mp, K, xh, rs, st);
+        if (slots <= 1024u) return launch_lines<XBF16, LAYOUT, 8, 4, 2, false>(x, M, Mp, K, xh, rs, st);
+        return launch_lines<XBF16, LAYOUT, 12, 4, 2, false>(x, M, Mp, K, xh, rs, st);
     }
-    if (slots <= 64u) hipLaunchKernelGGL((xprep_kernel<XBF16, LAYOUT, 1>), grid, block, 0, st, x, M, Mp, K, xh, rs);
-    else if (slots <= 128u) hipLaunchKernelGGL((xprep_kernel<XBF16, LAYOUT, 2>), grid, block, 0, st, x, M, Mp, K, xh, rs);
-    else if (slots <= 256u) hipLaunchKernelGGL((xprep_kernel<XBF16, LAYOUT, 4>), grid, block, 0, st, x, M, Mp, K, xh, rs);
-    else if (slots <= 512u) hipLaunchKernelGGL((xprep_kernel<XBF16, LAYOUT, 8>), grid, block, 0, st, x, M, Mp, K, xh, rs);
-    else if (slots <= 1024u) hipLaunchKernelGGL((xprep_kernel<XBF16, LAYOUT, 16>), grid, block, 0, st, x, M, Mp, K, xh, rs);
-    else if (slots <= 1536u) hipLaunchKernelGGL((xprep_kernel<XBF16, LAYOUT, 24>), grid, block, 0, st, x, M, Mp, K, xh, rs);
-    else hipLaunchKernelGGL((xprep_kernel<XBF16, LAYOUT, 0>), grid, block, 0, st, x, M, Mp, K, xh, rs);
-    return hipGetLastError();
+    if (Mp >= kXprepPartsMinRows && K >= kXprepPartsMinK) {
+        // slots per workgroup so that the launch has about 256 of them
+        const uint64_t want = ((uint64_t)slots * (Mp / kXprepLinesRows) + 255u) / 256u;
+        if (want <= 64u) return launch_lines<XBF16, LAYOUT, 1, 1, 1, true>(x, M, Mp, K, xh, rs, st);
+        if (want <= 128u) return launch_lines<XBF16, LAYOUT, 1, 1, 2, true>(x, M, Mp, K, xh, rs, st);
+        if (want <= 256u) return launch_lines<XBF16, LAYOUT, 2, 2, 2, true>(x, M, Mp, K, xh, rs, st);
+        return launch_lines<XBF16, LAYOUT, 4, 4, 2, true>(x, M, Mp, K, xh, rs, st);
+    }
+    // waves per row: 4096 waves in all (16 per CU), at least one slot per lane, at most eight
+    const uint32_t full = (K + 511u) / 512u;  // waves with one slot per lane
+    uint32_t wpr = 1u;
+    while (wpr < 16u && ((wpr < full && wpr * Mp < 4096u) || 8u * wpr < full)) wpr *= 2u;
+    switch (wpr) {
+        case 1: return launch_rows<XBF16, LAYOUT, 1>(x, M, Mp, K, xh, rs, st);
+        case 2: return launch_rows<XBF16, LAYOUT, 2>(x, M, Mp, K, xh, rs, st);
+        case 4: return launch_rows<XBF16, LAYOUT, 4>(x, M, Mp, K, xh, rs, st);
+        case 8: return launch_rows<XBF16, LAYOUT, 8>(x, M, Mp, K, xh, rs, st);
+        default: return launch_rows<XBF16, LAYOUT, 16>(x, M, Mp, K, xh, rs, st);
+    }
 }
 
 template <uint32_t LAYOUT>
