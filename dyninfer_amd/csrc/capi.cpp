@@ -230,20 +230,21 @@ bool has_prefill_gemm(uint32_t enc, uint32_t N, uint32_t K, uint32_t rows, bool 
     return rows >= min_rows && dmx::gemm_supported(enc, N, K, rows);
 }
 
-// The prefill path: x staged once (xprep), then one GEMM per weight.
+// The prefill path: x staged once (xprep), then one GEMM launch for all weights.
 hipError_t prefill(const dyninfer_qweight_t* ws, uint32_t count, const void* x, uint32_t x_dtype, uint32_t rows,
                    void* const* ys, uint32_t y_dtype, uint8_t* work, hipStream_t st) {
     const uint32_t K = (uint32_t)ws[0].cols;
     uint16_t* xh = reinterpret_cast<uint16_t*>(work);
     float* rs = reinterpret_cast<float*>(work + dmx::prefill_xh_bytes(rows, K));
     const uint32_t enc = ws[0].encoding;
-    hipError_t e = dmx::xprep_launch(x, x_dtype == DYNINFER_DTYPE_BF16, rows, K, dmx::gemm_layout(enc), xh, rs, st);
-    for (uint32_t i = 0; i < count && e == hipSuccess; i++) {
-        const dmx::GemmWeight wt{enc, static_cast<const uint8_t*>(ws[i].data), static_cast<const uint8_t*>(ws[i].scales),
-                                 static_cast<const uint8_t*>(ws[i].biases), ws[i].group_size, ws[i].scale_dtype};
-        e = dmx::gemm_launch(wt, (uint32_t)ws[i].rows, K, xh, rs, rows, ys[i], y_dtype == DYNINFER_DTYPE_BF16, st);
-    }
-    return e;
+    const hipError_t e = dmx::xprep_launch(x, x_dtype == DYNINFER_DTYPE_BF16, rows, K, dmx::gemm_layout(enc), xh, rs, st);
+    if (e != hipSuccess) return e;
+    dmx::GemmWeight wts[dmx::kMaxProblems];
+    for (uint32_t i = 0; i < count; i++)
+        wts[i] = {enc, static_cast<const uint8_t*>(ws[i].data), static_cast<const uint8_t*>(ws[i].scales),
+                  static_cast<const uint8_t*>(ws[i].biases), ws[i].group_size, ws[i].scale_dtype, (uint32_t)ws[i].rows,
+                  ys[i]};
+    return dmx::gemm_launch(wts, (int)count, K, xh, rs, rows, y_dtype == DYNINFER_DTYPE_BF16, st);
 }
 
 // Runs rows > 16 through the GEMV kernels 16 activation rows at a time (the

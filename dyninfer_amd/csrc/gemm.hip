@@ -18,30 +18,17 @@ extern template hipError_t launch_plan<ENC_MLX_U4>(const GemmArgs&, const GemmPl
 
 namespace {
 
-bool fits_enc(uint32_t enc, int tm, int nb, int s) {
+bool fits_enc(uint32_t enc, uint32_t tm, uint32_t nb, uint32_t s, uint32_t wn, uint32_t wm) {
     switch (enc) {
-        case ENC_Q4_0: return fits<ENC_Q4_0>(tm, nb, s);
-        case ENC_Q4_1: return fits<ENC_Q4_1>(tm, nb, s);
-        case ENC_Q8_0: return fits<ENC_Q8_0>(tm, nb, s);
-        case ENC_Q6_K: return fits<ENC_Q6_K>(tm, nb, s);
-        case ENC_Q4_K: return fits<ENC_Q4_K>(tm, nb, s);
-        case ENC_Q5_K: return fits<ENC_Q5_K>(tm, nb, s);
-        case ENC_IQ4_XS: return fits<ENC_IQ4_XS>(tm, nb, s);
-        case ENC_MLX_U4: return fits<ENC_MLX_U4>(tm, nb, s);
+        case ENC_Q4_0: return fits<ENC_Q4_0>(tm, nb, s, wn, wm);
+        case ENC_Q4_1: return fits<ENC_Q4_1>(tm, nb, s, wn, wm);
+        case ENC_Q8_0: return fits<ENC_Q8_0>(tm, nb, s, wn, wm);
+        case ENC_Q6_K: return fits<ENC_Q6_K>(tm, nb, s, wn, wm);
+        case ENC_Q4_K: return fits<ENC_Q4_K>(tm, nb, s, wn, wm);
+        case ENC_Q5_K: return fits<ENC_Q5_K>(tm, nb, s, wn, wm);
+        case ENC_IQ4_XS: return fits<ENC_IQ4_XS>(tm, nb, s, wn, wm);
+        case ENC_MLX_U4: return fits<ENC_MLX_U4>(tm, nb, s, wn, wm);
         default: return false;
-    }
-}
-
-// Decode VALU instructions per (N-block, k step) per lane, from the kernels'
-// ISA: the encoding's term in the cost model.
-double dec_cost(uint32_t enc) {
-    switch (enc) {
-        case ENC_Q8_0: return 18.0;
-        case ENC_Q6_K: return 30.0;
-        case ENC_Q4_K: return 22.0;
-        case ENC_Q5_K:
-        case ENC_IQ4_XS: return 28.0;
-        default: return 16.0;  // Q4_0, Q4_1, MLX U4
     }
 }
 
@@ -55,9 +42,9 @@ uint32_t gemm_layout(uint32_t enc) {
         case ENC_Q4_0:
         case ENC_Q4_1: return XFRAG_NIB;
         case ENC_Q8_0: return XFRAG_BYTE;
-        case ENC_Q6_K: return XFRAG_BYTE;  // a lane's 32 codes in order, as Q8_0
+        case ENC_Q6_K: return XFRAG_Q6K;
         case ENC_Q4_K:
-        case ENC_Q5_K: return XFRAG_BYTE;
+        case ENC_Q5_K: return XFRAG_QK;
         case ENC_IQ4_XS: return XFRAG_NIB;  // a sub-block laid out as a Q4_0 block
         case ENC_MLX_U4: return XFRAG_WORD;
         default: return ~0u;
@@ -69,66 +56,78 @@ bool gemm_supported(uint32_t enc, uint32_t N, uint32_t K, uint32_t M) {
            K % (enc == ENC_Q6_K || enc == ENC_Q4_K || enc == ENC_Q5_K || enc == ENC_IQ4_XS ? 256u : 64u) == 0;
 }
 
-// Launch plan from a cost model fitted to graph-replayed calls (staging +
-// GEMM) of every plan on 17 shapes (M 128..2048, N 1024..12288, K 1024..12288;
-// Q4_0, Q6_K, Q4_K, Q8_0, MLX U4), in us per call:
-//   t = 3.87 + rounds · (nc · (0.0712·TM·NB + 0.2074·NB·dec/16 + 0.0737)
-//                        + 0.0987·TM·NB·(S > 1 ? 4 : 1) + 4.99)
-// with nc the 64-k chunks per wave (K/64/S), rounds = ceil(workgroups / 256)
-// (one workgroup per CU), dec the encoding's decode VALU per (N-block, k
-// step); the last term is the epilogue's LDS round trip of the partial tiles.
-// It picks the measured best plan on 16 of the 17 shapes and one within 1.2%
-// on the other (MLX M512 N3072 K1024).  Candidates: TM 2 or 4 activation row
-// blocks (4 only above 64 rows), NB 2 or 3 weight row blocks per wave, S 1, 2
-// or 4 K slices per workgroup (those whose LDS fits, S dividing the chunks).
-GemmPlan gemm_plan(uint32_t enc, uint32_t N, uint32_t K, uint32_t M) {
-    const double dec = gemm::dec_cost(enc) / 16.0;
+// Launch plan from a cost model fitted to graph-replayed launches of every
+// configuration on 86 shapes of each of six encodings (M 20..2048, N 1024..24576, K
+// 768..12288; Q4_0, Q6_K, Q5_K, Q8_0, IQ4_XS, MLX U4), in us:
+//   t = 0.86 + wg·(1 + r·(rounds - 1)),
+//   wg = 1.04 + 0.101·TM·NB·S' + nc·(0.00165·V + 0.0673·TM·NB + 0.38)·(1 + 0.37·(w - 1)),
+// with rounds = ceil(workgroups / 256), nc the 64-k chunks per wave, V the decode and
+// scale VALU of a chunk, w waves per SIMD, S' = S (the epilogue's LDS round trip of
+// the partial tiles), r = 0.75 where several workgroups fit a CU (small tiles of four
+// waves), otherwise 1.  The configuration it picks takes 0.9% longer on average than the best
+// of them (8% at the 95th percentile, 18% at worst).
+GemmPlan gemm_plan(uint32_t enc, const uint32_t* N, int count, uint32_t K, uint32_t M) {
     const uint32_t mb = (M + 31u) / 32u, nchk = K / 64u;
-    GemmPlan best{2, 2, 1, 0, 0};
+    const double valu = 4.0 * gemm::decode_valu(enc) + gemm::scale_valu(enc);
+    GemmPlan best{};
     double best_t = 1e300;
-    for (uint32_t tm : {4u, 2u}) {
-        if (tm == 4u && mb <= 2u) continue;
-        for (uint32_t nb : {3u, 2u}) {
-            for (uint32_t s : {4u, 2u, 1u}) {
-                if (!gemm::fits_enc(enc, (int)tm, (int)nb, (int)s) || nchk % s != 0) continue;
-                const uint32_t wn = 4u / s;
-                const uint32_t mt = (mb + tm - 1u) / tm, nt = (N + 32u * nb * wn - 1u) / (32u * nb * wn);
-                const double nc = (double)(nchk / s), rounds = (double)(((uint64_t)mt * nt + 255u) / 256u);
-                const double t = 3.87 + rounds * (nc * (0.0712 * tm * nb + 0.2074 * nb * dec + 0.0737) +
-                                                   0.0987 * tm * nb * (s > 1u ? 4.0 : 1.0) + 4.99);
-                if (t < best_t * 0.999) {
-                    best_t = t;
-                    best = {tm, nb, s, mt, nt};
-                }
-            }
+    auto consider = [&](uint32_t tm, uint32_t nb, uint32_t s, uint32_t wn, uint32_t wm) {
+        // slices that share slots are equal; a slice holds at least one chunk
+        if (!gemm::fits_enc(enc, tm, nb, s, wn, wm) || (wn * wm > 1u ? nchk % s != 0 : nchk < s)) return;
+        if (nchk >= 4u && tm * wm > 1u && tm * wm / 2u >= mb) return;  // half the rows would do
+        uint32_t nt = 0;
+        for (int i = 0; i < count; i++) nt += (N[i] + 32u * nb * wn - 1u) / (32u * nb * wn);
+        const uint32_t mt = (mb + tm * wm - 1u) / (tm * wm);
+        const double nc = (double)((nchk + s - 1u) / s), rounds = (double)(((uint64_t)mt * nt + 255u) / 256u);
+        const double w = s * wn * wm / 4.0, tiles = tm * nb;
+        const double wg = 1.04 + 0.101 * tiles * s +
+                          nc * (0.00165 * nb * valu + 0.0673 * tiles + 0.38) * (1.0 + 0.37 * (w - 1.0));
+        const double t = 0.86 + wg * (1.0 + (tiles <= 4.0 && tm <= 2u && w == 1.0 ? 0.75 : 1.0) * (rounds - 1.0));
+        if (t < best_t * 0.999) {
+            best_t = t;
+            best = {tm, nb, s, wn, wm, mt, nt};
         }
-    }
+    };
+#define X(TM, NB, S, WN, WM) consider(TM, NB, S, WN, WM);
+    DMX_GEMM_CONFIGS(X)
+#undef X
     return best;
 }
 
-hipError_t gemm_launch(const GemmWeight& wt, uint32_t N, uint32_t K, const uint16_t* xh, const float* rs, uint32_t M,
-                       void* y, bool y_bf16, hipStream_t st) {
-    const uint32_t enc = wt.enc;
-    if (!gemm_supported(enc, N, K, M)) return hipErrorInvalidValue;
-    if (enc == ENC_MLX_U4 && (wt.group == 0 || wt.group % 32u || K % wt.group || wt.sdtype > DT_BF16 || !wt.sc || !wt.bi))
-        return hipErrorInvalidValue;
-    const GemmPlan p = gemm_plan(enc, N, K, M);
+hipError_t gemm_launch(const GemmWeight* wts, int count, uint32_t K, const uint16_t* xh, const float* rs, uint32_t M,
+                       bool y_bf16, hipStream_t st) {
+    if (count < 1 || count > kMaxProblems) return hipErrorInvalidValue;
+    const GemmWeight& w0 = wts[0];
+    const uint32_t enc = w0.enc;
+    uint32_t N[kMaxProblems];
+    uint64_t ntotal = 0;
+    for (int i = 0; i < count; i++) {
+        const GemmWeight& wt = wts[i];
+        if (wt.enc != enc || !gemm_supported(enc, wt.N, K, M)) return hipErrorInvalidValue;
+        if (enc == ENC_MLX_U4 && (wt.group == 0 || wt.group % 32u || K % wt.group || wt.group != w0.group ||
+                                  wt.sdtype != w0.sdtype || wt.sdtype > DT_BF16 || !wt.sc || !wt.bi))
+            return hipErrorInvalidValue;
+        N[i] = wt.N;
+        ntotal += wt.N;
+    }
+    const GemmPlan p = gemm_plan(enc, N, count, K, M);
+    if (p.tm == 0) return hipErrorInvalidConfiguration;
     GemmArgs a{};
-    a.w = wt.w;
     a.xh = xh;
     a.rs = rs;
-    a.y = y;
     a.M = M;
-    a.N = N;
     a.K = K;
     a.mt = p.mt;
     a.nt = p.nt;
     a.y_bf16 = y_bf16 ? 1u : 0u;
-    a.sc = wt.sc;
-    a.bi = wt.bi;
-    a.group = wt.group;
-    a.gmagic = group_magic(wt.group);
-    a.sdtype = wt.sdtype;
+    a.group = w0.group;
+    a.gmagic = group_magic(w0.group);
+    a.sdtype = w0.sdtype;
+    a.np = (uint32_t)count;
+    for (int i = 0, nt0 = 0; i < count; i++) {
+        a.p[i] = {wts[i].w, wts[i].sc, wts[i].bi, wts[i].y, wts[i].N, (uint32_t)nt0};
+        nt0 += (int)((wts[i].N + 32u * p.nb * p.wn - 1u) / (32u * p.nb * p.wn));
+    }
     switch (enc) {
         case ENC_Q4_0: a.rowbytes = (uint64_t)(K / 32u) * 18u; break;
         case ENC_Q4_1: a.rowbytes = (uint64_t)(K / 32u) * 20u; break;
@@ -141,7 +140,7 @@ hipError_t gemm_launch(const GemmWeight& wt, uint32_t N, uint32_t K, const uint1
     }
     // M-major tile order when the staged activations (2 bytes per element)
     // outweigh the weights (M2048 N3072 K1024: 34.3 against 35.9 us per call)
-    a.mmajor = (uint64_t)M * K * 2u > (uint64_t)N * a.rowbytes ? 1u : 0u;
+    a.mmajor = (uint64_t)M * K * 2u > ntotal * a.rowbytes ? 1u : 0u;
     switch (enc) {
         case ENC_Q4_0: return gemm::launch_plan<ENC_Q4_0>(a, p, st);
         case ENC_Q4_1: return gemm::launch_plan<ENC_Q4_1>(a, p, st);

@@ -142,8 +142,12 @@ hipError_t gather_launch(uint32_t enc, const uint8_t* w, const uint8_t* sc, cons
 // 32.  Lane half h of k step 4c + t holds 8 k of k = 64c + 32h + (0..31):
 enum XFrag : uint32_t {
     XFRAG_NIB = 2,   // Q4_0, Q4_1: 4t, 4t+2, 4t+1, 4t+3, 16+4t, 18+4t, 17+4t, 19+4t
-    XFRAG_BYTE = 3,  // Q8_0, Q6_K, Q4_K: 8t + (0, 2, 1, 3, 4, 6, 5, 7)
+    XFRAG_BYTE = 3,  // Q8_0:       8t + (0, 2, 1, 3, 4, 6, 5, 7)
     XFRAG_WORD = 4,  // MLX U4:     8t + (0, 4, 1, 5, 2, 6, 3, 7)
+    // k relative to the chunk (QK) or, with c the chunk's number, to its super-block
+    // of four chunks (Q6K), in BYTE's order:
+    XFRAG_QK = 5,    // Q4_K, Q5_K: 16h + 32·(t / 2) + 8·(t % 2) + (0, 2, 1, 3, 4, 6, 5, 7)
+    XFRAG_Q6K = 6,   // Q6_K:       128·(c / 2 % 2) + 16·(c % 2) + 32h + 64·(t / 2) + 8·(t % 2) + ...
 };
 hipError_t xprep_launch(const void* x, bool x_bf16, uint32_t M, uint32_t K, uint32_t layout, uint16_t* xh, float* rs,
                         hipStream_t stream);
@@ -158,17 +162,19 @@ inline uint64_t prefill_workspace_bytes(uint32_t M, uint32_t K) {
     return prefill_xh_bytes(M, K) + (((uint64_t)M + 255u) & ~(uint64_t)255u) * 4u;
 }
 
-// Prefill GEMM launch plan (gemm.hip): workgroups of four waves, each owning a
-// (32·tm) x (32·nb·4/s) tile of Y, the waves split over s K slices.
+// Prefill GEMM launch plan (gemm.hip): workgroups of s·wn waves, each owning a
+// (32·tm) x (32·nb·wn) tile of one weight's Y, the waves split over s K slices
+// and wn column subtiles.
 struct GemmPlan {
-    uint32_t tm, nb, s;
-    uint32_t mt, nt;  // workgroup tiles along M and N
+    uint32_t tm, nb, s, wn, wm;
+    uint32_t mt, nt;  // workgroup tiles along M and (every weight's) along N
 };
-GemmPlan gemm_plan(uint32_t enc, uint32_t N, uint32_t K, uint32_t M);
+GemmPlan gemm_plan(uint32_t enc, const uint32_t* N, int count, uint32_t K, uint32_t M);
 
-// Prefill GEMM on MFMA (gemm.hip): Y[M, N] = diag(rs) · (Xh[M, K] · Wᵀ), Xh/rs
-// from xprep_launch(gemm_layout(enc)); Y f32 or bf16.  gemm_layout returns ~0u
-// for encodings without a GEMM.  The weight: GGUF blocks at w, or MLX U4
+// Prefill GEMM on MFMA (gemm.hip): y_i[M, N_i] = diag(rs) · (Xh[M, K] · W_iᵀ) for
+// i < count weights of one encoding (group, scale dtype) and K in one launch, Xh/rs
+// from xprep_launch(gemm_layout(enc)); y_i f32 or bf16.  gemm_layout returns ~0u
+// for encodings without a GEMM.  A weight: GGUF blocks at w, or MLX U4
 // packed words at w with scales sc and biases bi [N, K/group] of dtype sdtype.
 struct GemmWeight {
     uint32_t enc;
@@ -176,10 +182,12 @@ struct GemmWeight {
     const uint8_t* sc;
     const uint8_t* bi;
     uint32_t group, sdtype;
+    uint32_t N;
+    void* y;
 };
 uint32_t gemm_layout(uint32_t enc);
 bool gemm_supported(uint32_t enc, uint32_t N, uint32_t K, uint32_t M);
-hipError_t gemm_launch(const GemmWeight& wt, uint32_t N, uint32_t K, const uint16_t* xh, const float* rs, uint32_t M,
-                       void* y, bool y_bf16, hipStream_t stream);
+hipError_t gemm_launch(const GemmWeight* wts, int count, uint32_t K, const uint16_t* xh, const float* rs, uint32_t M,
+                       bool y_bf16, hipStream_t stream);
 
 }  // namespace dmx

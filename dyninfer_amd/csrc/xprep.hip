@@ -21,12 +21,17 @@
 // k = 64c + 32h .. 64c + 32h + 31, in the order the block's decode produces:
 //   XFRAG_NIB  (Q4_0, Q4_1: code byte j holds k = j and k = j + 16):
 //              4t, 4t+2, 4t+1, 4t+3, 16+4t, 18+4t, 17+4t, 19+4t
-//   XFRAG_BYTE (Q8_0, Q6_K: one code byte per k):
+//   XFRAG_BYTE (Q8_0: one code byte per k):
 //              8t, 8t+2, 8t+1, 8t+3, 8t+4, 8t+6, 8t+5, 8t+7
 //              (pairs (j, j+2) of a dword decode together)
 //   XFRAG_WORD (MLX U4: packed word t of the block holds k = 8t .. 8t+7, LSB
 //              first): 8t, 8t+4, 8t+1, 8t+5, 8t+2, 8t+6, 8t+3, 8t+7
-//              (nibbles j and j+4 of a word decode together).  Rows M .. roundup(M, 32) - 1
+//              (nibbles j and j+4 of a word decode together)
+// and for the super-block encodings, whose lane half takes both nibbles of 16
+// code bytes (runs of 8 k in XFRAG_BYTE's order, k0 their first):
+//   XFRAG_QK   (Q4_K, Q5_K): k0 = 64c + 16h + 32·(t / 2) + 8·(t % 2)
+//   XFRAG_Q6K  (Q6_K): k0 = 256·(c / 4) + 128·(c / 2 % 2) + 16·(c % 2) + 32h +
+//              64·(t / 2) + 8·(t % 2).  Rows M .. roundup(M, 32) - 1
 // are written as zeros, so the GEMM reads whole fragments.
 //
 // Mapping: a row is shared by WPR waves, each lane taking up to NR output slots
@@ -58,10 +63,13 @@ typedef float xf2 __attribute__((ext_vector_type(2)));
 typedef float xf4 __attribute__((ext_vector_type(4)));
 
 // The 8 activations of output slot `slot` of a row: two runs of 4 k, at
-// k0 and k0 + RUN2 (NIB: 16, BYTE and WORD: 4, i.e. one run of 8).
+// k0 and k0 + RUN2 (NIB: 16, the others 4, i.e. one run of 8).
 template <uint32_t LAYOUT>
 __device__ __forceinline__ uint32_t slot_k0(uint32_t slot) {
     const uint32_t c = slot >> 3, t = (slot >> 1) & 3u, h = slot & 1u;
+    if (LAYOUT == XFRAG_QK) return 64u * c + 16u * h + 32u * (t >> 1) + 8u * (t & 1u);
+    if (LAYOUT == XFRAG_Q6K)
+        return 256u * (c >> 2) + 128u * ((c >> 1) & 1u) + 16u * (c & 1u) + 32u * h + 64u * (t >> 1) + 8u * (t & 1u);
     return 64u * c + 32u * h + (LAYOUT == XFRAG_NIB ? 4u * t : 8u * t);
 }
 template <bool XBF16, uint32_t LAYOUT>
@@ -109,7 +117,7 @@ __device__ __forceinline__ size_t frag_offset(uint32_t m, uint32_t slot, uint32_
     return (((size_t)(m >> 5) * ksteps + 4u * c + t) * 64u + (m & 31u) + 32u * h) * 8u;
 }
 
-// NIB and BYTE pair (v0, v2), (v1, v3), (v4, v6), (v5, v7); WORD pairs (v0, v4),
+// All but WORD pair (v0, v2), (v1, v3), (v4, v6), (v5, v7); WORD pairs (v0, v4),
 // (v1, v5), (v2, v6), (v3, v7).
 typedef uint32_t xu4 __attribute__((ext_vector_type(4)));
 template <uint32_t LAYOUT>
@@ -348,6 +356,8 @@ hipError_t xprep_launch(const void* x, bool x_bf16, uint32_t M, uint32_t K, uint
         case XFRAG_NIB: return launch_xprep<XFRAG_NIB>(x, x_bf16, M, K, xh, rs, st);
         case XFRAG_BYTE: return launch_xprep<XFRAG_BYTE>(x, x_bf16, M, K, xh, rs, st);
         case XFRAG_WORD: return launch_xprep<XFRAG_WORD>(x, x_bf16, M, K, xh, rs, st);
+        case XFRAG_QK: return launch_xprep<XFRAG_QK>(x, x_bf16, M, K, xh, rs, st);
+        case XFRAG_Q6K: return launch_xprep<XFRAG_Q6K>(x, x_bf16, M, K, xh, rs, st);
         default: return hipErrorInvalidValue;
     }
 }

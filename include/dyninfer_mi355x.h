@@ -137,7 +137,7 @@ const char* dyninfer_mi355x_last_error(void);
  *     of 64 (256 for the super-block
  *     encodings): x is staged once per call as f16 MFMA operand fragments,
  *     each row scaled by a power of two (RNE) and the rows padded with zeros to a
- *     multiple of 32, into the caller's workspace; then one MFMA GEMM per weight
+ *     multiple of 32, into the caller's workspace; then one MFMA GEMM launch
  *     decodes the GGUF blocks or MLX words straight into MFMA operands.  Every other
  *     case (K not a multiple of 64, Q4_0, Q6_K, Q4_K, Q5_K and IQ4_XS at 17..32 rows
  *     with K <= 8192) runs the GEMV kernels over 16-row chunks.
@@ -177,7 +177,7 @@ int dyninfer_mi355x_qlinear(dyninfer_mi355x_ctx_t* ctx, const dyninfer_qweight_t
  * Several weights that share one activation (q/k/v, gate/up) in a single launch:
  * y_i = x · W_iᵀ for i < count.  All weights must have the same encoding (and group
  * size / scale dtype) and the same K; N may differ.  count <= 4, any rows (prefill
- * stages x once and runs one GEMM per weight).
+ * stages x once and runs one GEMM launch over all of them).
  * No reference counterpart as one call: the reference emits one helper call per
  * linear (parameter.rs:141-183); this is the same arithmetic batched into one launch.
  */

@@ -1,0 +1,86 @@
+"""GPU parity for every configuration the prefill GEMM's planner picks (tile, K split,
+shared or own activation fragments), each encoding, against the CPU oracle: ragged rows
+and columns, several weights in one launch, K slices that differ by a chunk (K = 320,
+1088, 1280), slices of one chunk.
+
+Tolerances, as max over outputs of |y - y64| / sum_k |w||x|: 2^-10 + 2e-5 (one f16
+rounding of each weight and activation, plus f32 accumulation); Q6_K and IQ4_XS weights
+round twice (+ 2^-11); Q4_K and Q5_K weights are RNE_f16(q RNE_f16(d sc) -
+RNE_f16(dmin m)), three roundings of terms that may nearly cancel, bounded through
+sum_k |dmin m||x|."""
+import numpy as np
+import pytest
+import torch
+
+import dyninfer_amd as d
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+BLOCKS = ["q4_0", "q4_1", "q8_0", "mlx_u4"]
+SUPER = ["q6_k", "q4_k", "q5_k", "iq4_xs"]
+
+
+def weight(kind, n, k, seed):
+    """(QWeight, dequantised weights, |min| of each weight) of synthetic blocks."""
+    if kind == "mlx_u4":
+        packed, sc, bi = oracle.synth_mlx_u4(n, k, 64, oracle.D_BF16, seed=seed)
+        t = [torch.from_numpy(a).cuda() for a in (packed, sc, bi)]
+        return (d.QWeight(d.ENC_MLX_U4, n, k, *t, 64, d.DTYPE_BF16),
+                oracle.dequant_mlx_u4(packed, sc, bi, oracle.D_BF16, n, k, 64), None)
+    g = getattr(oracle, kind.upper())
+    data = oracle.synth_gguf(g, n, k, seed)
+    w = d.QWeight(getattr(d, "ENC_" + kind.upper()), n, k, torch.from_numpy(data).cuda())
+    wf = oracle.dequant_gguf(g, data, n, k)
+    if kind not in ("q4_k", "q5_k"):
+        return w, wf, None
+    zero = data.reshape(-1, 144 if kind == "q4_k" else 176).copy()
+    zero[:, 16:] = 0  # every code 0: the weights are -dmin m
+    return w, wf, np.abs(oracle.dequant_gguf(g, zero.reshape(-1), n, k))
+
+
+def check(ctx, kind, m, ns, k):
+    made = [weight(kind, n, k, seed=m + n + k) for n in ns]
+    x = oracle.randn(m * k, seed=m + k).reshape(m, k)
+    xd = torch.from_numpy(x).cuda()
+    ys = ctx.qlinear_multi([w for w, _, _ in made], xd) if len(ns) > 1 else [ctx.qlinear(made[0][0], xd)]
+    pick = np.unique(np.concatenate([np.arange(min(m, 3)), np.arange(max(m - 3, 0), m), np.arange(0, m, 61)]))
+    for y, (_, wf, mins) in zip(ys, made):
+        y64, absdot = oracle.linear_f64(x[pick], wf)
+        tol = 2.0 ** -10 + 2e-5 + (2.0 ** -11 if kind in SUPER else 0.0)
+        bound = tol * absdot
+        if mins is not None:
+            bound = bound + 2.0 ** -10 * (np.abs(x[pick]).astype(np.float64) @ mins.T.astype(np.float64))
+        err = np.abs(y.cpu().numpy()[pick].astype(np.float64) - y64)
+        assert (err <= bound).all(), float((err / absdot).max())
+
+
+# (rows, weight rows, K): the configuration (TM, NB, S, WN, WM) the planner picks for most encodings
+SHAPES = [
+    (33, [97], 256),            # 1 1 4 1 1, a chunk per slice
+    (45, [131, 62], 1280),      # 1 1 8 1 1, slices of 2 and 3 chunks
+    (33, [4000, 101], 256),     # 2 1 4 1 1
+    (50, [9001], 512),          # 2 2 4 1 1
+    (75, [8000, 900, 103], 256),  # 2 3 4 1 1
+    (70, [14001], 512),         # 4 2 4 1 1
+    (97, [19000, 1001], 768),   # 4 3 4 1 1
+    (131, [13000, 1003], 768),  # 8 2 4 1 1
+    (131, [9001], 256),         # 2 2 1 4 1
+    (257, [14002], 256),        # 4 2 1 2 2
+    (400, [20001], 256),        # 8 2 1 4 1
+    (400, [20001], 1024),       # the two above over a ring's worth of chunks
+    (513, [6000, 3001], 1280),
+]
+
+
+@pytest.mark.parametrize("kind", BLOCKS + SUPER)
+@pytest.mark.parametrize("m,ns,k", SHAPES, ids=[f"{m}-{'+'.join(map(str, ns))}-{k}" for m, ns, k in SHAPES])
+def test_gemm_plans(ctx, kind, m, ns, k):
+    check(ctx, kind, m, ns, k)
+
+
+@pytest.mark.parametrize("kind", BLOCKS)
+@pytest.mark.parametrize("m,ns,k", [(40, [97], 64), (41, [260, 30], 192), (70, [513], 320), (90, [1000], 1088),
+                                    (300, [20000], 64)])
+def test_gemm_plans_odd_chunks(ctx, kind, m, ns, k):
+    check(ctx, kind, m, ns, k)
