@@ -51,15 +51,16 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
 
 constexpr uint32_t kMagic = 0x64006400u;  // f16 1024.0 in both halves
 
-// (a & m) | b as one v_and_or_b32.  Written as asm because the compiler
-// otherwise emits v_and_b32 + v_or_b32 with literal operands (a VOP3 op takes
-// no literal on gfx9).  The mask lives in a scalar register and b in a vector
-// register (gfx9 allows one scalar operand per VALU instruction), both loaded
-// once outside the loops.
+// (a & m) | b as one v_and_or_b32: the mask in a scalar register and b in a vector
+// register (gfx9 allows one scalar operand per VALU instruction and a VOP3 op no
+// literal), both loaded once outside the loops.  The constants pass through empty
+// asm so that the compiler does not fold them into v_and_b32 + v_or_b32 with literals;
+// the instruction itself is the compiler's, which knows the wait states an MFMA
+// needs after a VALU write of its operand (written as asm, it gave MFMAs stale pairs).
 __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t m, uint32_t b) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(m), "v"(b));
-    return r;
+    asm("" : "+s"(m));
+    asm("" : "+v"(b));
+    return (a & m) | b;
 }
 
 // Selector for v_perm_b32 that extracts the dword starting `sh` bytes into a

@@ -111,6 +111,28 @@ hipError_t launch(uint32_t enc, const GemvParams& p, uint32_t B, uint32_t onesho
 
 }  // namespace
 
+// Whether a launch of 3..8 rows that the 16-row MFMA GEMV could serve runs the 4x4
+// MFMA kernels instead (chunk_dot4): 3..4 rows, all but Q6_K from 4096 tiles of 16
+// rows (151936 x 4096: 112 us on the 16-row path against 117); 5..8 rows, launches
+// below 8 MB and 1024 tiles (Q6_K 1024 x 4096 at 8 rows 9.4 -> 7.4 us; Q4_K 4096 x
+// 4096, 9.4 MB, 9.8 us on the 16-row path against 10.9).
+static bool gemv_prefers_4x4(uint32_t enc, const GemvProblem* probs, int nprob, uint32_t batch, uint32_t K) {
+    if (batch > 8u) return false;
+    uint64_t tiles = 0, rows = 0;
+    for (int i = 0; i < nprob; i++) {
+        tiles += (probs[i].n + 15u) / 16u;
+        rows += probs[i].n;
+    }
+    if (batch <= 4u) return enc != ENC_Q6_K || tiles < 4096u;
+    const uint64_t row = enc == ENC_Q4_0   ? K / 32u * 18u
+                         : enc == ENC_Q6_K ? K / 256u * 210u
+                         : enc == ENC_Q4_K ? K / 256u * 144u
+                         : enc == ENC_Q5_K ? K / 256u * 176u
+                         : enc == ENC_IQ4_XS ? K / 256u * 136u
+                                             : K / 2u;
+    return rows * row < (8ull << 20) && tiles < 1024u;
+}
+
 uint64_t gemv_workspace_bytes(uint32_t enc, const GemvProblem* probs, int nprob, uint32_t batch, uint32_t K,
                               bool y_bf16, uint32_t group) {
     if (nprob < 1 || nprob > kMaxProblems) return 0;
@@ -123,12 +145,14 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
     EncInfo info;
     if (!enc_info(enc, info) || nprob < 1 || nprob > kMaxProblems || batch < 1 || batch > (uint32_t)kMaxGemvBatch)
         return hipErrorInvalidValue;
-    // 5..16 activation rows: every weight decoded once for all rows, on MFMA
-    if (gemv_mfma_applies(enc, probs, nprob, batch, K, y_bf16, group))
+    // 9..16 activation rows, and 3..8 on large launches: every weight decoded once for
+    // all rows, on 16-row MFMAs
+    const bool m4 = gemv_prefers_4x4(enc, probs, nprob, batch, K);
+    if (!m4 && gemv_mfma_applies(enc, probs, nprob, batch, K, y_bf16, group))
         return gemv_mfma_launch(enc, probs, nprob, K, x, x_bf16, batch, y_bf16, group, sdtype, work, work_bytes,
                                 stream);
     // bf16 outputs and K in several segments: on MFMA when the workspace holds f32 accumulators
-    if (y_bf16 && work) {
+    if (!m4 && y_bf16 && work) {
         const uint64_t need = gemv_mfma_bf16_acc_bytes(enc, probs, nprob, batch, K, group);
         if (need && work_bytes >= need)
             return gemv_mfma_launch_bf16_acc(enc, probs, nprob, K, x, x_bf16, batch, group, sdtype, work, work_bytes,
@@ -164,20 +188,16 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
     // covers consecutive blocks; splitting a wave over distant rows costs DRAM
     // locality) and a row block's chunks need few rounds.  When L does not
     // divide the chunk count, the lanes past the last chunk add zero.
-    uint32_t L = 1;
-    while (L < 64 && 2 * L <= nch) L *= 2;
+    // 4 and 8 activation rows: sixteen lanes along K, four rows (4x4 MFMAs).
+    uint32_t L = B >= 4 ? 16 : 1;
+    while (B < 4 && L < 64 && 2 * L <= nch) L *= 2;
     uint32_t lanes_log2 = 0;
     while ((1u << lanes_log2) < L) lanes_log2++;
     // Latency mode (one wave per row block of one row per lane group, all of
     // a lane's chunks loaded at once) when the matrices give at most 16384
     // such row blocks and a lane few chunks: 4 for one activation row (64-
     // weight chunks: 2; at 3 the 8B down_proj ran slower than the pipeline,
-    // Q4_K 4096 x 12288 12.6 against 9.1 us), 2 for 2 and 8 rows (at 8 rows
-    // the Qwen3-0.6B MLX step 853 -> 744 us per launch set, q/k/v 6.9 -> 5.5
-    // us, down 8.1 -> 7.7; 2 chunks take ~300 registers there, so that kernel
-    // runs in 256-thread workgroups only), 1 for 4 (64-weight
-    // chunks: at most 2048 row blocks; 12288 x 4096 Q4_K 28.6 us against 17.7
-    // us in the pipeline, 1024 x 4096 6.3 against 6.7 us).  64-weight chunks
+    // Q4_K 4096 x 12288 12.6 against 9.1 us), 2 for 2 rows.  64-weight chunks
     // at 2 rows: at most 4096 row blocks at 1 chunk per lane and 2048 at 2
     // (per launch, Q4_K/Q5_K/Q6_K 13824 x 5120: 30.4/32.1/32.0 us in latency
     // mode against 18.9/22.1/21.7 in the pipeline, 12288 x 4096 13.7 against
@@ -190,9 +210,30 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
     uint64_t rbs1 = 0;
     for (int i = 0; i < nprob; i++) rbs1 += (probs[i].n + (64u >> lanes_log2) - 1) / (64u >> lanes_log2);
     const uint32_t cpl = (nch + L - 1) >> lanes_log2;
-    const uint32_t max_cpl = B == 1 ? (info.wide ? 2u : 4u) : B == 2 ? 2u : B == 4 ? 1u : B == 8 ? 2u : 0u;
-    const uint64_t max_rbs = !info.wide || B == 1 ? 16384u : B == 4 ? 2048u : cpl == 1 ? 4096u : 2048u;
-    const uint32_t oneshot = cpl >= 1 && cpl <= max_cpl && rbs1 <= max_rbs ? cpl : 0u;
+    const uint32_t max_cpl = B == 1 ? (info.wide ? 2u : 4u) : 2u;
+    const uint64_t max_rbs = !info.wide || B == 1 ? 16384u : cpl == 1 ? 4096u : 2048u;
+    uint32_t oneshot = cpl >= 1 && cpl <= max_cpl && rbs1 <= max_rbs ? cpl : 0u;
+    if (B >= 4) {
+        // 4 and 8 rows, a row block being four rows by sixteen lanes.  Up to 512 row
+        // blocks (1024 at 4 rows from K = 2048) one wave each would leave most SIMDs
+        // idle: four waves share one (us per launch, one wave against four: MLX 1024 x
+        // 3072 at 8 rows 8.8 -> 6.5, Q8_0 10.8 -> 8.6, Q6_K 1024 x 4096 at 4 rows 7.6
+        // -> 5.1, Q4_0 4096 x 4096 at 4 rows 6.5 -> 6.2; but 4096 x 1024 4.1 -> 4.8 and
+        // 4096 x 4096 at 8 rows 9.7 -> 11.9: every workgroup stages the activations).
+        // Where the activations leave one workgroup per CU it has 1024 threads (Q4_0
+        // 4096 x 12288 at 4 rows 17.3 -> 15.0; 64-weight chunks spill there).  One
+        // wave per row block up to 8192 of them at 1..2 chunks per lane (MLX 6144 x
+        // 1024 at 8 rows 5.8 us in the pipeline, 5.3) and 2048 at more (Q4_0 6144 x
+        // 4096 at 4 rows 10.2 against 8.0; Q4_0 24576 x 4096 16.4 against 20.5).
+        const uint64_t tile = xtile_bytes(enc, B, K);
+        const uint32_t cps = (nch + 63u) / 64u;  // chunks per lane, four waves per row block
+        if (cps <= 2u && tile + kSplitSums <= lim && (rbs1 <= 512u || (B == 4u && rbs1 <= 1024u && K >= 2048u)))
+            oneshot = kOneshotSplit | cps;
+        else if (!info.wide && B == 4u && rbs1 <= 2048u && tile > kLdsBytes / 2u && tile + kSplitSums <= lim && cps <= 8u)
+            oneshot = kOneshotWide | (cps <= 4u ? 4u : 8u);
+        else if (cpl <= 2u) oneshot = rbs1 <= 8192u ? cpl : 0u;
+        else oneshot = rbs1 <= 2048u && cpl <= (info.wide ? 4u : 8u) ? (cpl <= 4u ? 4u : 8u) : 0u;
+    }
 
     GemvParams p = {};
     for (int i = 0; i < kMaxProblems; i++) {

@@ -1,5 +1,5 @@
-// Decode GEMV kernel templates (activation rows 1..16) for GGUF Q4_0/Q4_1/Q8_0/
-// Q6_K and MLX affine U4.
+// Decode GEMV kernel templates (activation rows 1..16) for the GGUF encodings and MLX
+// affine U4.
 //
 // Semantics: y[b, o] = Σ_k x[b, k] · w[o, k] with f32 accumulation, w the
 // reference's dequantised weight (gguf_codegen.rs:268-314 `emit_linear`,
@@ -24,7 +24,8 @@
 //     activation loads (before the staging arithmetic), so HBM latency
 //     overlaps staging and arithmetic;
 //   * per weight: half a v_and_or_b32 and half a v_dot2_f32_f16 per
-//     activation row; per group and row: two or three f32 ops;
+//     activation row (4 and 8 rows: a sixteenth of a 4x4x4 MFMA per four rows,
+//     chunk_dot4); per group and row: two or three f32 ops;
 //   * at the end of a row block the L lanes combine their R·B partial sums
 //     with cross-lane shuffles and lane 0 of the group stores.
 // Several weights that share one activation (q/k/v, gate/up) are served by one
@@ -71,6 +72,37 @@ struct XTile {
     static constexpr uint32_t chunk_bytes = XPW * 4 + E::NG * NCF * 4;
     static_assert(chunk_bytes == xtile_chunk_bytes(E::ENC), "host/device activation tile layouts differ");
 };
+
+// Kernels of 4 or 8 activation rows multiply on 4x4 MFMAs (chunk_dot4): the tile's
+// rows are skewed by 16 bytes (four lanes read one chunk of four rows at a time) and
+// the constants of one (chunk, group) lie together, f32 [nch][NG][NCF][B].
+template <int B>
+constexpr bool kM4 = B >= 4;
+template <class E, int B>
+__device__ __forceinline__ uint32_t xrow_dwords(uint32_t nch) {
+    return nch * XTile<E>::XPW + (kM4<B> ? kXRowSkew / 4u : 0u);
+}
+template <class E, int B>
+__device__ __forceinline__ const float* xconsts(const uint8_t* lds, uint32_t nch) {
+    return reinterpret_cast<const float*>(lds) + (size_t)B * xrow_dwords<E, B>(nch);
+}
+// Stores (-C, s, s·Σx) of (row b, chunk u, group g).
+template <class E, int B>
+__device__ __forceinline__ void store_consts(uint8_t* lds, uint32_t nch, uint32_t b, uint32_t u, uint32_t g, float negc,
+                                             float s, float sm) {
+    using XT = XTile<E>;
+    float* xc = const_cast<float*>(xconsts<E, B>(lds, nch));
+    if constexpr (kM4<B>) {
+        float* c = xc + (size_t)(u * E::NG + g) * (XT::NCF * B) + b;
+        c[0] = negc;
+        c[B] = s;
+        if constexpr (XT::NCF == 4) c[2 * B] = sm;
+    } else {
+        float* c = xc + ((size_t)(b * nch + u) * E::NG + g) * XT::NCF;
+        if constexpr (XT::NCF == 4) *reinterpret_cast<float4*>(c) = make_float4(negc, s, sm, 0.0f);
+        else *reinterpret_cast<float2*>(c) = make_float2(negc, s);
+    }
+}
 
 // Activations off..off+3 of the source as f32 (f32 or bf16 source).  off is a
 // multiple of 4 and rows start 16-byte aligned, so this is one aligned 16-byte
@@ -159,7 +191,7 @@ struct GStage {
     static constexpr int TT = E::NT / SP;                   // code dwords per thread
     static constexpr int RPG = E::NG == 1 ? E::NXR : 1;     // runs of 4 per code dword in one group
     float v[TT][RPG][4];
-    uint32_t item;  // b·nch + u
+    uint32_t b, u;  // activation row, chunk
     uint32_t g;     // scale group within the chunk
     uint32_t q;     // part of the group (code dwords q·TT ..)
     bool live;      // the group exists: the thread stores
@@ -176,8 +208,10 @@ __device__ __forceinline__ void gstage_load(const GemvParams& p, uint32_t nch, u
     s.live = gi0 < groups;
     const uint32_t gi = s.live ? gi0 : groups - 1u;  // spare lanes redo the last group, unstored
     s.g = E::NG == 1 ? 0u : gi % (uint32_t)E::NG;
-    s.item = E::NG == 1 ? gi : gi / (uint32_t)E::NG;
-    const uint32_t b = B == 1 ? 0u : s.item / nch, u = s.item - b * nch;
+    const uint32_t item = E::NG == 1 ? gi : gi / (uint32_t)E::NG;
+    const uint32_t b = B == 1 ? 0u : item / nch, u = item - b * nch;
+    s.b = b;
+    s.u = u;
     // Rows past the batch restage row 0: in bounds, and their sums are never
     // stored.  Activation offsets are 32-bit (the activations are < 4 GiB).
     const uint32_t base = (b < p.batch ? b : 0u) * p.ldx + E::xbase(u) + (uint32_t)E::RUNSTRIDE * s.g +
@@ -239,8 +273,8 @@ __device__ __forceinline__ void gstage_store(uint8_t* lds, uint32_t nch, const G
     float St = 0.0f;
     if constexpr (XT::NCF == 4) St = __uint_as_float(sp_reduce<SP>(__float_as_uint(Sx[0] + Sx[1]), fadd));
     if (s.live) {
-        uint32_t* xp = reinterpret_cast<uint32_t*>(lds) + (size_t)s.item * XT::XPW + s.q * (uint32_t)(S::TT * E::PPT);
-        float* xc = reinterpret_cast<float*>(lds + (size_t)B * nch * XT::XPW * 4u);
+        uint32_t* xp = reinterpret_cast<uint32_t*>(lds) + s.b * xrow_dwords<E, B>(nch) + s.u * XT::XPW +
+                       s.q * (uint32_t)(S::TT * E::PPT);
         if constexpr (E::NG == 1 && (S::TT * E::PPT) % 4 == 0) {
             // the thread's pairs are TT·PPT consecutive dwords
 #pragma unroll
@@ -260,12 +294,7 @@ __device__ __forceinline__ void gstage_store(uint8_t* lds, uint32_t nch, const G
         }
         if (s.q == 0) {
             const float sc = ldexpf(1.0f, ex - 14);
-            float* c = xc + ((size_t)s.item * E::NG + s.g) * XT::NCF;
-            if constexpr (XT::NCF == 4) {
-                *reinterpret_cast<float4*>(c) = make_float4(-Ct, sc, sc * St, 0.0f);
-            } else {
-                *reinterpret_cast<float2*>(c) = make_float2(-Ct, sc);
-            }
+            store_consts<E, B>(lds, nch, s.b, s.u, s.g, -Ct, sc, sc * St);
         }
     }
 }
@@ -310,8 +339,8 @@ __device__ __forceinline__ void stage_x_sp(uint8_t* lds, const GemvParams& p, MI
 template <class E>
 struct XStage {
     float v[E::NXR][4];
-    uint32_t item;
-    bool live;  // item < B·nch: the thread stores
+    uint32_t b, u;  // activation row, chunk
+    bool live;      // the thread stores
 };
 
 // Issues the loads of staging thread idx (no use of the loaded values, so
@@ -321,8 +350,10 @@ __device__ __forceinline__ void xstage_load(const GemvParams& p, uint32_t nch, u
     const uint32_t items = (uint32_t)B * nch;
     const uint32_t it = idx / (uint32_t)E::NT, t = idx % (uint32_t)E::NT;
     s.live = it < items;
-    s.item = s.live ? it : items - 1u;  // spare threads redo the last chunk, unstored
-    const uint32_t b = B == 1 ? 0u : s.item / nch, u = s.item - b * nch;
+    const uint32_t item = s.live ? it : items - 1u;  // spare threads redo the last chunk, unstored
+    const uint32_t b = B == 1 ? 0u : item / nch, u = item - b * nch;
+    s.b = b;
+    s.u = u;
     // Rows past the batch restage row 0: in bounds, and their sums are never
     // stored.  Activation offsets are 32-bit (the activations are < 4 GiB).
     const uint32_t base = (b < p.batch ? b : 0u) * p.ldx + E::xbase(u) + (uint32_t)E::TSTRIDE * t;
@@ -341,7 +372,6 @@ __device__ __forceinline__ void xstage_store(uint8_t* lds, uint32_t nch, uint32_
     using XT = XTile<E>;
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     uint32_t* xp = reinterpret_cast<uint32_t*>(lds);
-    float* xc = reinterpret_cast<float*>(lds + (size_t)B * nch * XT::XPW * 4u);
     auto val = [&](int h, int e) -> float {
         const int r = xrun_of<E>(h, e);
         return s.v[r][E::xoff(0, h, e) - E::xrun0(r)];
@@ -396,7 +426,7 @@ __device__ __forceinline__ void xstage_store(uint8_t* lds, uint32_t nch, uint32_
         if constexpr (XT::NCF == 4) S[g] = __uint_as_float(lanes_reduce<E::NT>(__float_as_uint(S[g]), fadd));
     }
     if (s.live) {
-        uint32_t* dst = xp + (size_t)s.item * XT::XPW + t * (uint32_t)E::PPT;
+        uint32_t* dst = xp + s.b * xrow_dwords<E, B>(nch) + s.u * XT::XPW + t * (uint32_t)E::PPT;
         if constexpr (E::PPT % 4 == 0) {
 #pragma unroll
             for (int h = 0; h < E::PPT; h += 4)
@@ -409,12 +439,7 @@ __device__ __forceinline__ void xstage_store(uint8_t* lds, uint32_t nch, uint32_
 #pragma unroll
             for (int g = 0; g < E::NG; g++) {
                 const float sc = ldexpf(1.0f, ex[g] - 14);
-                float* c = xc + ((size_t)s.item * E::NG + g) * XT::NCF;
-                if constexpr (XT::NCF == 4) {
-                    *reinterpret_cast<float4*>(c) = make_float4(-C[g], sc, sc * S[g], 0.0f);
-                } else {
-                    *reinterpret_cast<float2*>(c) = make_float2(-C[g], sc);
-                }
+                store_consts<E, B>(lds, nch, s.b, s.u, (uint32_t)g, -C[g], sc, sc * S[g]);
             }
         }
     }
@@ -422,25 +447,38 @@ __device__ __forceinline__ void xstage_store(uint8_t* lds, uint32_t nch, uint32_
 
 // Stages activation rows [0, batch) into the tile (rows up to B restage row 0),
 // one thread per code dword: B·nch·NT staging threads, P per workgroup thread
-// per round.  The first round's activation loads are issued, then mid() (the
-// caller's first weight loads), then the first round is computed: loads
-// return in issue order, so the activations arrive ahead of the weights and
-// the staging arithmetic runs while the weights are in flight.  Later rounds
-// (large batches) load after the weights.  Ends with a barrier.
+// per round.  A round's activation loads are issued, then mid() (the caller's
+// first weight loads), then the round is computed: loads return in issue
+// order, so the activations arrive ahead of the weights and the staging
+// arithmetic runs while the weights are in flight.  mid() goes into the first
+// round, and at 4 rows into the last: a later round's activations would queue
+// behind the weights, which cost latency mode with its many weight loads most
+// (Q4_0 4096 x 12288 at 4 rows 23.3 -> 15.0 us; the pipeline 18.8 -> 17.3).
+// Ends with a barrier.
 template <class E, int B, bool XBF16, int P, int TH, class MID>
 __device__ __forceinline__ void stage_x_rounds(uint8_t* lds, const GemvParams& p, MID&& mid) {
     const uint32_t nch = p.K / (uint32_t)E::CW;
     const uint32_t total = (uint32_t)B * nch * (uint32_t)E::NT;
     const uint32_t t = threadIdx.x % (uint32_t)E::NT;  // the workgroup size is a multiple of NT
     XStage<E> s[P];
+    uint32_t base = 0;
+    if constexpr (B == 4) {
+        for (; base + (uint32_t)P * TH < total; base += (uint32_t)P * TH) {
 #pragma unroll
-    for (int ps = 0; ps < P; ps++) xstage_load<E, B, XBF16>(p, nch, threadIdx.x + (uint32_t)ps * TH, s[ps]);
+            for (int ps = 0; ps < P; ps++)
+                xstage_load<E, B, XBF16>(p, nch, base + threadIdx.x + (uint32_t)ps * TH, s[ps]);
+#pragma unroll
+            for (int ps = 0; ps < P; ps++) xstage_store<E, B>(lds, nch, t, s[ps]);
+        }
+    }
+#pragma unroll
+    for (int ps = 0; ps < P; ps++) xstage_load<E, B, XBF16>(p, nch, base + threadIdx.x + (uint32_t)ps * TH, s[ps]);
     __builtin_amdgcn_sched_barrier(0);
     mid();
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ps = 0; ps < P; ps++) xstage_store<E, B>(lds, nch, t, s[ps]);
-    for (uint32_t base = (uint32_t)P * TH; base < total; base += (uint32_t)P * TH) {
+    for (base += (uint32_t)P * TH; base < total; base += (uint32_t)P * TH) {
 #pragma unroll
         for (int ps = 0; ps < P; ps++)
             xstage_load<E, B, XBF16>(p, nch, base + threadIdx.x + (uint32_t)ps * TH, s[ps]);
@@ -551,10 +589,10 @@ __device__ __forceinline__ void load_consts(const float* xc, uint32_t idx, float
     }
 }
 
-// The PPT activation pairs of code dword t of chunk u, activation row b.
+// The PPT activation pairs of code dword t of the chunk at xp.
 template <class E>
-__device__ __forceinline__ void load_xpairs(const uint32_t* xp, uint32_t idx, int t, uint32_t (&xv)[E::PPT]) {
-    const uint32_t* xq = xp + (size_t)idx * XTile<E>::XPW + t * E::PPT;
+__device__ __forceinline__ void load_xpairs(const uint32_t* xp, int t, uint32_t (&xv)[E::PPT]) {
+    const uint32_t* xq = xp + t * E::PPT;
     if constexpr (E::PPT % 4 == 0) {
 #pragma unroll
         for (int h = 0; h < E::PPT; h += 4) {
@@ -568,98 +606,127 @@ __device__ __forceinline__ void load_xpairs(const uint32_t* xp, uint32_t idx, in
     }
 }
 
-// y[i][b] += Σ over chunk u of row i: w·x, for R rows and B activation rows.
-// Up to 4 activation rows: code dword outer (each dword's pairs are decoded
-// and used at once, R·B·NG accumulators).  More rows: activation row outer
-// (the chunk's pairs are decoded once and kept, R·NG accumulators), which
-// keeps the registers of the wide batches in check.
+// y[i][b] += Σ over chunk u of row i: w·x, for R rows and B activation rows (up to
+// 2; code dword outer: each dword's pairs are decoded and used at once, R·B·NG
+// accumulators).
 template <class E, int R, int B>
 __device__ __forceinline__ void chunk_dot(const typename E::Chunk (&c)[R], const uint8_t* lds, uint32_t nch,
                                           uint32_t u, float (&y)[R][B]) {
-    using XT = XTile<E>;
     const uint32_t* xp = reinterpret_cast<const uint32_t*>(lds);
-    const float* xc = reinterpret_cast<const float*>(lds + (size_t)B * nch * XT::XPW * 4u);
-    if constexpr (B <= 4) {
-        float acc[R][B][E::NG];
-        float sc[B][E::NG], sm[B][E::NG];
+    const float* xc = xconsts<E, B>(lds, nch);
+    float acc[R][B][E::NG];
+    float sc[B][E::NG], sm[B][E::NG];
+#pragma unroll
+    for (int b = 0; b < B; b++)
+#pragma unroll
+        for (int g = 0; g < E::NG; g++) {
+            float negc;
+            load_consts<E>(xc, ((uint32_t)b * nch + u) * E::NG + g, negc, sc[b][g], sm[b][g]);
+#pragma unroll
+            for (int i = 0; i < R; i++) acc[i][b][g] = negc;
+        }
+#pragma unroll
+    for (int t = 0; t < E::NT; t++) {
+        uint32_t pr[R][E::PPT];
+#pragma unroll
+        for (int i = 0; i < R; i++) E::pairs(c[i], t, pr[i]);
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            uint32_t xv[E::PPT];
+            load_xpairs<E>(xp + ((uint32_t)b * nch + u) * XTile<E>::XPW, t, xv);
+#pragma unroll
+            for (int i = 0; i < R; i++)
+#pragma unroll
+                for (int h = 0; h < E::PPT; h++) {
+                    float& a = acc[i][b][E::grp(t, h)];
+                    a = dot2(pr[i][h], xv[h], a);
+                }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < R; i++)
 #pragma unroll
         for (int b = 0; b < B; b++)
 #pragma unroll
             for (int g = 0; g < E::NG; g++) {
-                float negc;
-                load_consts<E>(xc, ((uint32_t)b * nch + u) * E::NG + g, negc, sc[b][g], sm[b][g]);
-#pragma unroll
-                for (int i = 0; i < R; i++) acc[i][b][g] = negc;
+                // weight scale first: d·acc·s is the group's true contribution,
+                // while acc·s alone (Σ q·x) can overflow f32 for huge activations
+                y[i][b] = fmaf(E::gscale(c[i], g) * acc[i][b][g], sc[b][g], y[i][b]);
+                if constexpr (E::AFFINE) y[i][b] = fmaf(E::goffset(c[i], g), sm[b][g], y[i][b]);
             }
+}
+
+// The same for 4 or 8 activation rows on v_mfma_f32_4x4x4_16b_f16: sixteen 4x4 products
+// of depth 4 an instruction, one per block of four lanes.  The four lanes of a block
+// hold the same chunk u of four weight rows (operand B: lane j two decoded pairs of
+// row j) and two pairs of four activation rows (operand A: lane i those of row i, so
+// a lane reads one activation row from LDS instead of B); every lane ends with its
+// own weight row's sums for the four activation rows.  Same products and constants
+// as chunk_dot; per 32 Q4_0 weights and 4 rows, 8 MFMAs of 8 cycles (beside the
+// VALU) and 5 LDS reads in place of 64 v_dot2 and 20.  us per launch, v_dot2 or the
+// 16-row MFMA path against this: at 4 rows Q4_K 24576 x 4096 24.0 -> 19.7, 5120 x 4096
+// 12.8 -> 8.9, Q4_0 24576 x 4096 21.2 -> 17.0, MLX 151936 x 1024 33.9 -> 25.5; at 8
+// rows Q8_0 12288 x 4096 107 -> 20.4 (registers), MLX 6144 x 1024 6.9 -> 5.3.  Bound
+// now by the staging each workgroup does and the decode, not by the products.
+template <class E, int R, int B>
+__device__ __forceinline__ void chunk_dot4(const typename E::Chunk (&c)[R], const uint8_t* lds, uint32_t nch,
+                                           uint32_t u, float (&y)[R][B]) {
+    using XT = XTile<E>;
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    constexpr int BB = B / 4;
+    const uint32_t* xp = reinterpret_cast<const uint32_t*>(lds) + (threadIdx.x & 3u) * xrow_dwords<E, B>(nch) + u * XT::XPW;
+    const float* xc = xconsts<E, B>(lds, nch) + (size_t)u * (E::NG * XT::NCF * B);
+    f32x4 acc[R][BB][E::NG];
 #pragma unroll
-        for (int t = 0; t < E::NT; t++) {
-            uint32_t pr[R][E::PPT];
+    for (int q = 0; q < BB; q++)
 #pragma unroll
-            for (int i = 0; i < R; i++) E::pairs(c[i], t, pr[i]);
+        for (int g = 0; g < E::NG; g++) {
+            const f32x4 negc = *reinterpret_cast<const f32x4*>(xc + (g * XT::NCF) * B + 4 * q);
 #pragma unroll
-            for (int b = 0; b < B; b++) {
-                uint32_t xv[E::PPT];
-                load_xpairs<E>(xp, (uint32_t)b * nch + u, t, xv);
-#pragma unroll
-                for (int i = 0; i < R; i++)
-#pragma unroll
-                    for (int h = 0; h < E::PPT; h++) {
-                        float& a = acc[i][b][E::grp(t, h)];
-                        a = dot2(pr[i][h], xv[h], a);
-                    }
-            }
+            for (int i = 0; i < R; i++) acc[i][q][g] = negc;
         }
 #pragma unroll
-        for (int i = 0; i < R; i++)
+    for (int t = 0; t < E::NT; t++) {
+        uint32_t pr[R][E::PPT];
 #pragma unroll
-            for (int b = 0; b < B; b++)
+        for (int i = 0; i < R; i++) E::pairs(c[i], t, pr[i]);
 #pragma unroll
-                for (int g = 0; g < E::NG; g++) {
-                    // weight scale first: d·acc·s is the group's true contribution,
-                    // while acc·s alone (Σ q·x) can overflow f32 for huge activations
-                    y[i][b] = fmaf(E::gscale(c[i], g) * acc[i][b][g], sc[b][g], y[i][b]);
-                    if constexpr (E::AFFINE) y[i][b] = fmaf(E::goffset(c[i], g), sm[b][g], y[i][b]);
+        for (int q = 0; q < BB; q++) {
+            uint32_t xv[E::PPT];
+            load_xpairs<E>(xp + 4 * q * xrow_dwords<E, B>(nch), t, xv);
+            // pairs h and h2 of one scale group
+#pragma unroll
+            for (int h = 0; h < E::PPT; h++) {
+                constexpr int D = E::NG == 1 ? 1 : E::NG;
+                if (E::NG == 1 ? (h & 1) != 0 : h >= E::NG) continue;
+                const int h2 = h + D;
+                const h4 a = __builtin_bit_cast(h4, u32x2{xv[h], xv[h2]});
+#pragma unroll
+                for (int i = 0; i < R; i++) {
+                    f32x4& s = acc[i][q][E::grp(t, h)];
+                    s = __builtin_amdgcn_mfma_f32_4x4x4f16(a, __builtin_bit_cast(h4, u32x2{pr[i][h], pr[i][h2]}), s, 0, 0, 0);
                 }
-    } else {
-        uint32_t pr[R][E::NT][E::PPT];
-#pragma unroll
-        for (int i = 0; i < R; i++)
-#pragma unroll
-            for (int t = 0; t < E::NT; t++) E::pairs(c[i], t, pr[i][t]);
-#pragma unroll
-        for (int b = 0; b < B; b++) {
-            float acc[R][E::NG], sc[E::NG], sm[E::NG];
-#pragma unroll
-            for (int g = 0; g < E::NG; g++) {
-                float negc;
-                load_consts<E>(xc, ((uint32_t)b * nch + u) * E::NG + g, negc, sc[g], sm[g]);
-#pragma unroll
-                for (int i = 0; i < R; i++) acc[i][g] = negc;
             }
+        }
+    }
 #pragma unroll
-            for (int t = 0; t < E::NT; t++) {
-                uint32_t xv[E::PPT];
-                load_xpairs<E>(xp, (uint32_t)b * nch + u, t, xv);
+    for (int q = 0; q < BB; q++)
 #pragma unroll
-                for (int i = 0; i < R; i++)
-#pragma unroll
-                    for (int h = 0; h < E::PPT; h++) {
-                        float& a = acc[i][E::grp(t, h)];
-                        a = dot2(pr[i][t][h], xv[h], a);
-                    }
-            }
+        for (int g = 0; g < E::NG; g++) {
+            const f32x4 sc = *reinterpret_cast<const f32x4*>(xc + (g * XT::NCF + 1) * B + 4 * q);
+            f32x4 sm = {0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (E::AFFINE) sm = *reinterpret_cast<const f32x4*>(xc + (g * XT::NCF + 2) * B + 4 * q);
 #pragma unroll
             for (int i = 0; i < R; i++)
 #pragma unroll
-                for (int g = 0; g < E::NG; g++) {
-                    y[i][b] = fmaf(E::gscale(c[i], g) * acc[i][g], sc[g], y[i][b]);
-                    if constexpr (E::AFFINE) y[i][b] = fmaf(E::goffset(c[i], g), sm[g], y[i][b]);
+                for (int r = 0; r < 4; r++) {
+                    float& o = y[i][4 * q + r];
+                    o = fmaf(E::gscale(c[i], g) * acc[i][q][g][r], sc[r], o);
+                    if constexpr (E::AFFINE) o = fmaf(E::goffset(c[i], g), sm[r], o);
                 }
-            // one activation row's LDS reads in flight at a time: hoisting all of
-            // them (which the optimiser does before scheduling) would spill
-            asm volatile("" ::: "memory");
         }
-    }
 }
 
 // Row block -> its problem's pointers, row count and first row (all wave-
@@ -709,13 +776,21 @@ __device__ __forceinline__ float group_sum(float v, uint32_t L) {
     return v;
 }
 
+// Sum over the sixteen lanes of a wave with the same lane % 4, in every lane.
+__device__ __forceinline__ float stride4_sum(float v) {
+#define DMX_DPP(x, ctrl) __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xF, 0xF, false))
+    v += DMX_DPP(v, 0x124);  // row_ror:4
+    v += DMX_DPP(v, 0x128);  // row_ror:8
+#undef DMX_DPP
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 template <int R, int B>
-__device__ __forceinline__ void reduce_store(float (&acc)[R][B], const RowBlock& rb, uint32_t row0, uint32_t j,
-                                             uint32_t L, const GemvParams& p) {
-#pragma unroll
-    for (int i = 0; i < R; i++)
-#pragma unroll
-        for (int b = 0; b < B; b++) acc[i][b] = group_sum(acc[i][b], L);
+__device__ __forceinline__ void store_sums(const float (&acc)[R][B], const RowBlock& rb, uint32_t row0, uint32_t j,
+                                           const GemvParams& p) {
     if (j == 0) {
         void* y = rb.y;
 #pragma unroll
@@ -734,6 +809,16 @@ __device__ __forceinline__ void reduce_store(float (&acc)[R][B], const RowBlock&
             }
         }
     }
+}
+
+template <int R, int B>
+__device__ __forceinline__ void reduce_store(float (&acc)[R][B], const RowBlock& rb, uint32_t row0, uint32_t j,
+                                             uint32_t L, const GemvParams& p) {
+#pragma unroll
+    for (int i = 0; i < R; i++)
+#pragma unroll
+        for (int b = 0; b < B; b++) acc[i][b] = kM4<B> ? stride4_sum(acc[i][b]) : group_sum(acc[i][b], L);
+    store_sums<R, B>(acc, rb, row0, j, p);
 }
 
 // The persistent task pipeline shared by all encodings.  load(rb, row, u)
@@ -770,7 +855,8 @@ __device__ __forceinline__ void gemv_pipeline(const GemvParams& p, const uint8_t
     // dispatch packet that the first weight loads would wait behind.
     const uint32_t wid = __builtin_amdgcn_readfirstlane(blockIdx.x * (uint32_t)(TH / 64) + (threadIdx.x >> 6));
     const uint32_t L = 1u << p.lanes_log2;
-    const uint32_t j = lane & (L - 1u), g = lane >> p.lanes_log2;
+    // (4x4 MFMAs: the four rows of a chunk on adjacent lanes, L = 16)
+    const uint32_t j = kM4<B> ? lane >> 2 : lane & (L - 1u), g = kM4<B> ? lane & 3u : lane >> p.lanes_log2;
     const uint32_t rows_per_rb = (64u >> p.lanes_log2) * (uint32_t)R;
     const uint32_t nch = p.K / (uint32_t)E::CW;
     const uint32_t cpl = (nch + L - 1u) >> p.lanes_log2;  // chunks per lane per row block
@@ -834,7 +920,8 @@ __device__ __forceinline__ void gemv_pipeline(const GemvParams& p, const uint8_t
             ch[i] = E::unpack(buf[i], u);
             E::zero_if(ch[i], past);
         }
-        chunk_dot<E, R, B>(ch, lds, nch, u, acc);
+        if constexpr (kM4<B>) chunk_dot4<E, R, B>(ch, lds, nch, u, acc);
+        else chunk_dot<E, R, B>(ch, lds, nch, u, acc);
         if (c + 1 == cpl) {
             reduce_store<R, B>(acc, blk, blk.base + g * (uint32_t)R, j, L, p);
 #pragma unroll
@@ -872,40 +959,66 @@ __device__ __forceinline__ void gemv_pipeline(const GemvParams& p, const uint8_t
 // launch waits on one memory latency; then it multiplies them for the B
 // activation rows, the L lanes reduce, and lane 0 stores.  TH is the
 // workgroup size.
-template <class E, int CPL, int B, int TH, class LOAD, class STAGE>
+//
+// KS > 1 (4 or 8 activation rows, few row blocks): KS waves of a workgroup share a
+// row block, each taking every KS-th run of L chunks, and the first adds their sums
+// from LDS.
+template <class E, int CPL, int B, int KS, int TH, class LOAD, class STAGE>
 __device__ __forceinline__ void gemv_oneshot(const GemvParams& p, const uint8_t* lds, LOAD&& load, STAGE&& stage) {
+    static_assert(KS == 1 || kM4<B>, "K split: 4 or 8 activation rows");
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wid = __builtin_amdgcn_readfirstlane(blockIdx.x * (uint32_t)(TH / 64) + (threadIdx.x >> 6));
+    const uint32_t rb = wid / (uint32_t)KS, ks = wid % (uint32_t)KS;
     const uint32_t L = 1u << p.lanes_log2;
-    const uint32_t j = lane & (L - 1u), g = lane >> p.lanes_log2;
+    // (4x4 MFMAs: the four rows of a chunk on adjacent lanes, L = 16)
+    const uint32_t j = kM4<B> ? lane >> 2 : lane & (L - 1u), g = kM4<B> ? lane & 3u : lane >> p.lanes_log2;
     const uint32_t rows_per_rb = 64u >> p.lanes_log2;
     const uint32_t nch = p.K / (uint32_t)E::CW;
-    const bool active = wid < p.total_rb;
-    const RowBlock blk = row_block(p, active ? wid : p.total_rb - 1u, rows_per_rb);
+    const bool active = rb < p.total_rb;
+    const RowBlock blk = row_block(p, active ? rb : p.total_rb - 1u, rows_per_rb);
     const uint32_t row = blk.base + g < blk.n ? blk.base + g : blk.n - 1u;
     typename E::Raw buf[CPL];
     stage([&] {
 #pragma unroll
         for (int c = 0; c < CPL; c++) {
-            const uint32_t u = j + (uint32_t)c * L;
+            const uint32_t u = j + ((uint32_t)(c * KS) + ks) * L;
             buf[c] = load(blk, row, u < nch ? u : nch - 1u);
         }
     });
-    if (!active) return;
+    if (KS == 1 && !active) return;
     float acc[1][B];
 #pragma unroll
     for (int b = 0; b < B; b++) acc[0][b] = 0.0f;
 #pragma unroll
     for (int c = 0; c < CPL; c++) {
-        const uint32_t u0 = j + (uint32_t)c * L;
+        const uint32_t u0 = j + ((uint32_t)(c * KS) + ks) * L;
         const bool past = u0 >= nch;  // a lane past the last chunk: adds zero
         const uint32_t u = past ? nch - 1u : u0;
         typename E::Chunk ch[1];
         ch[0] = E::unpack(buf[c], u);
         E::zero_if(ch[0], past);
-        chunk_dot<E, 1, B>(ch, lds, nch, u, acc);
+        if constexpr (kM4<B>) chunk_dot4<E, 1, B>(ch, lds, nch, u, acc);
+        else chunk_dot<E, 1, B>(ch, lds, nch, u, acc);
     }
-    reduce_store<1, B>(acc, blk, blk.base + g, j, L, p);
+    if constexpr (KS == 1) {
+        reduce_store<1, B>(acc, blk, blk.base + g, j, L, p);
+    } else {
+        __shared__ float part[TH / 64][4][B];
+        const uint32_t wave = threadIdx.x >> 6;
+#pragma unroll
+        for (int b = 0; b < B; b++) acc[0][b] = stride4_sum(acc[0][b]);
+        if (ks != 0 && lane < 4u)
+#pragma unroll
+            for (int b = 0; b < B; b++) part[wave][lane][b] = acc[0][b];
+        __syncthreads();
+        if (ks != 0 || !active) return;
+        if (lane < 4u)
+#pragma unroll
+            for (int k = 1; k < KS; k++)
+#pragma unroll
+                for (int b = 0; b < B; b++) acc[0][b] += part[wave + (uint32_t)k][lane][b];
+        store_sums<1, B>(acc, blk, blk.base + g, j, p);
+    }
 }
 
 // ---------------------------------------------------------------- GGUF
@@ -919,12 +1032,12 @@ __global__ __launch_bounds__(TH) void gguf_gemv_kernel(const GemvParams p) {
     gemv_pipeline<E, R, B, TH>(p, xlds, load, [&](auto&& mid) { stage_x_auto<E, B, XM, TH>(xlds, p, mid); });
 }
 
-template <class E, int CPL, int B, int XM, int TH>
+template <class E, int CPL, int B, int XM, int TH, int KS = 1>
 __global__ __launch_bounds__(TH) void gguf_gemv_oneshot_kernel(const GemvParams p) {
     extern __shared__ __align__(16) uint8_t xlds[];
     const uint32_t rowbytes = (p.K / (uint32_t)E::QK) * (uint32_t)E::BB;
     auto load = [&](const RowBlock& rb, uint32_t row, uint32_t u) { return E::load(rb.w, row * rowbytes, u); };
-    gemv_oneshot<E, CPL, B, TH>(p, xlds, load, [&](auto&& mid) { stage_x_auto<E, B, XM, TH>(xlds, p, mid); });
+    gemv_oneshot<E, CPL, B, KS, TH>(p, xlds, load, [&](auto&& mid) { stage_x_auto<E, B, XM, TH>(xlds, p, mid); });
 }
 
 // ---------------------------------------------------------------- MLX affine U4
@@ -962,10 +1075,10 @@ __global__ __launch_bounds__(TH) void mlx_u4_gemv_kernel(const GemvParams p) {
                                       [&](auto&& mid) { stage_x_auto<EncMlxU4, B, XM, TH>(xlds, p, mid); });
 }
 
-template <int CPL, int B, int XM, int TH>
+template <int CPL, int B, int XM, int TH, int KS = 1>
 __global__ __launch_bounds__(TH) void mlx_u4_gemv_oneshot_kernel(const GemvParams p) {
     extern __shared__ __align__(16) uint8_t xlds[];
-    gemv_oneshot<EncMlxU4, CPL, B, TH>(p, xlds, MlxLoad(p),
+    gemv_oneshot<EncMlxU4, CPL, B, KS, TH>(p, xlds, MlxLoad(p),
                                         [&](auto&& mid) { stage_x_auto<EncMlxU4, B, XM, TH>(xlds, p, mid); });
 }
 
@@ -1117,25 +1230,36 @@ int gemv_tiles(GemvTile* t, MK&& gemv_tile, uint32_t threads = kGemvThreads) {
 // them in 512-thread groups; measured on the Qwen3-0.6B projections (1,024
 // and 3,072 waves) 256 threads took 5-15% less time per launch, and on
 // launches that split evenly either way (2,048, 4,096, 6,144 waves) it cost
-// up to 12%.  A null k512 (a kernel built for 256 threads only) always
-// launches k256.
+// up to 12%.  ks: waves per row block.
 template <class KERNEL>
-hipError_t launch_oneshot(KERNEL k512, KERNEL k256, GemvParams p, size_t lds, hipStream_t st) {
+hipError_t launch_oneshot(KERNEL k512, KERNEL k256, GemvParams p, size_t lds, hipStream_t st, uint32_t ks = 1) {
     int cus = 0, per_cu = 0;
-    hipError_t e = k512 ? cached_occupancy(reinterpret_cast<const void*>(k512), lds, 512, &per_cu, &cus) : hipSuccess;
+    hipError_t e = cached_occupancy(reinterpret_cast<const void*>(k512), lds, 512, &per_cu, &cus);
     if (e != hipSuccess) return e;
     e = cached_occupancy(reinterpret_cast<const void*>(k256), lds, 256, &per_cu, &cus);
     if (e != hipSuccess) return e;
     if (cus < 1) return hipErrorInvalidConfiguration;
     layout_row_blocks(p, 64u >> p.lanes_log2);
+    const uint64_t all = (uint64_t)p.total_rb * ks;
     auto busiest = [&](uint32_t waves) {  // waves on the busiest CU, groups of `waves`
-        const uint64_t wgs = ((uint64_t)p.total_rb + waves - 1) / waves;
+        const uint64_t wgs = (all + waves - 1) / waves;
         return (wgs + (uint64_t)cus - 1) / (uint64_t)cus * waves;
     };
-    const bool small = !k512 || busiest(4) < busiest(8);
+    const bool small = busiest(4) < busiest(8);
     const uint32_t waves = small ? 4u : 8u;
-    p.grid = (p.total_rb + waves - 1) / waves;
+    p.grid = (uint32_t)((all + waves - 1) / waves);
     hipLaunchKernelGGL(small ? k256 : k512, dim3(p.grid), dim3(waves * 64u), lds, st, p);
+    return hipGetLastError();
+}
+
+// Latency mode with four waves per row block in workgroups of 1024 threads.
+inline hipError_t launch_oneshot_wide(GemvKernel k, GemvParams p, size_t lds, hipStream_t st) {
+    int cus = 0, per_cu = 0;
+    const hipError_t e = cached_occupancy(reinterpret_cast<const void*>(k), lds, 1024, &per_cu, &cus);
+    if (e != hipSuccess) return e;
+    layout_row_blocks(p, 64u >> p.lanes_log2);
+    p.grid = (p.total_rb + 3u) / 4u;
+    hipLaunchKernelGGL(k, dim3(p.grid), dim3(1024), lds, st, p);
     return hipGetLastError();
 }
 
@@ -1158,7 +1282,8 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
     }
     if (oneshot) {
         // chunks per lane (the host's limits): 1..4 for one activation row
-        // (64-weight chunks 1..2), 1..2 for 2 rows, 1 for 4
+        // (64-weight chunks 1..2), 1..2 for 2 rows, 1, 2, 4 or 8 (64-weight chunks:
+        // not 8) for 4 and 8
 #define DMX_ONESHOT(b, c)                                                                             \
     if (B == b && oneshot == c)                                                                       \
         return launch_oneshot(gguf_gemv_oneshot_kernel<E, c, b, xmode_rows(XM, b), 512>,                         \
@@ -1170,17 +1295,35 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
             DMX_ONESHOT(1, 3)
             DMX_ONESHOT(1, 4)
         }
-        if constexpr (max_register_batch(E::ENC) >= 2) {
-            DMX_ONESHOT(2, 1)
-            DMX_ONESHOT(2, 2)
+        DMX_ONESHOT(2, 1)
+        DMX_ONESHOT(2, 2)
+        DMX_ONESHOT(4, 1)
+        DMX_ONESHOT(4, 2)
+        DMX_ONESHOT(4, 4)
+        DMX_ONESHOT(8, 1)
+        DMX_ONESHOT(8, 2)
+        DMX_ONESHOT(8, 4)
+        // four waves per row block: kOneshotSplit besides the chunks per lane
+#define DMX_ONESHOT_SPLIT(b, c)                                                                       \
+    if (B == b && oneshot == (kOneshotSplit | c))                                                     \
+        return launch_oneshot(gguf_gemv_oneshot_kernel<E, c, b, xmode_rows(XM, b), 512, 4>,           \
+                              gguf_gemv_oneshot_kernel<E, c, b, xmode_rows(XM, b), 256, 4>, p, lds, st, 4u);
+#define DMX_ONESHOT_WIDE(c)                                                                           \
+    if (B == 4 && oneshot == (kOneshotWide | c))                                                      \
+        return launch_oneshot_wide(gguf_gemv_oneshot_kernel<E, c, 4, xmode_rows(XM, 4), 1024, 4>, p, lds, st);
+        DMX_ONESHOT_SPLIT(4, 1)
+        DMX_ONESHOT_SPLIT(4, 2)
+        DMX_ONESHOT_SPLIT(8, 1)
+        DMX_ONESHOT_SPLIT(8, 2)
+        if constexpr (!wide_chunks(E::ENC)) {
+            DMX_ONESHOT_WIDE(4)
+            DMX_ONESHOT_WIDE(8)
         }
-        if constexpr (max_register_batch(E::ENC) >= 4) DMX_ONESHOT(4, 1)
-        if constexpr (max_register_batch(E::ENC) >= 8) {
-            DMX_ONESHOT(8, 1)
-            // 8 rows of 2 chunks per lane take ~300 registers: 256-thread workgroups only
-            if (B == 8 && oneshot == 2)
-                return launch_oneshot<GemvKernel>(nullptr, gguf_gemv_oneshot_kernel<E, 2, 8, xmode_rows(XM, 8), 256>,
-                                                  p, lds, st);
+#undef DMX_ONESHOT_WIDE
+#undef DMX_ONESHOT_SPLIT
+        if constexpr (!wide_chunks(E::ENC)) {
+            DMX_ONESHOT(4, 8)
+            DMX_ONESHOT(8, 8)
         }
 #undef DMX_ONESHOT
         return hipErrorInvalidValue;
@@ -1199,10 +1342,8 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
     const bool big = B == 1 && p.K > 8192u;
 #define DMX_CASE(b)                                                                                            \
     case b:                                                                                                    \
-        if constexpr (b <= max_register_batch(E::ENC)) {                                                       \
-            n = gemv_tiles<E, b>(t, [](auto r) -> GemvKernel { return gguf_gemv_kernel<E, b, decltype(r)::value, xmode_rows(XM, b)>; }); \
-            n += gemv_tiles<E, b>(t + n, [](auto r) -> GemvKernel { return gguf_gemv_kernel<E, b, decltype(r)::value, xmode_rows(XM, b), 256>; }, 256u); \
-        }                                                                                                      \
+        n = gemv_tiles<E, b>(t, [](auto r) -> GemvKernel { return gguf_gemv_kernel<E, b, decltype(r)::value, xmode_rows(XM, b)>; }); \
+        n += gemv_tiles<E, b>(t + n, [](auto r) -> GemvKernel { return gguf_gemv_kernel<E, b, decltype(r)::value, xmode_rows(XM, b), 256>; }, 256u); \
         break;
     switch (B) {
     case 1:

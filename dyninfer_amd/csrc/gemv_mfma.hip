@@ -1180,8 +1180,11 @@ hipError_t launch_mode(MfmaParams p, uint32_t units, bool y_bf16, uint8_t* pre, 
 template <class M>
 int mfma_mode(uint32_t K, uint32_t tiles, bool y_bf16, uint32_t min_tiles);
 
+// Up to these rows a launch has another single-pass kernel, which small launches keep.
+uint32_t valu_pass_rows(uint32_t enc) { return wide_chunks(enc) ? 4u : 8u; }
+
 uint32_t mfma_min_tiles(uint32_t enc, uint32_t batch) {
-    return batch > max_register_batch(enc) ? kMfmaMinTilesTwoPasses : kMfmaMinTiles;
+    return batch > valu_pass_rows(enc) ? kMfmaMinTilesTwoPasses : kMfmaMinTiles;
 }
 
 template <class M>
@@ -1261,6 +1264,8 @@ bool gemv_mfma_applies(uint32_t enc, const GemvProblem* probs, int nprob, uint32
                                    : enc == ENC_Q5_K ? K / 256u * 176u
                                    : enc == ENC_IQ4_XS ? K / 256u * 136u
                                                      : K / 2u);
+    // (Launches of 3..8 rows that the 4x4 MFMA kernels run faster are taken out before,
+    // gemv.hip gemv_prefers_4x4; the figures here and below are against v_dot2 kernels.)
     // At 3-4 rows the VALU GEMV's per-row dot products are cheap enough that
     // only the largest launches gain, and Q4_0 (the cheapest MFMA decode) with
     // K = 4096 on 384-512 tiles: per launch at 4 rows, the 8B q/k/v (384 tiles)
@@ -1271,7 +1276,7 @@ bool gemv_mfma_applies(uint32_t enc, const GemvProblem* probs, int nprob, uint32
     // 6144 x 8192 15.8 -> 19.6 on MFMA).
     const bool q4_0_few = enc == ENC_Q4_0 && K == 4096u && tiles >= kMfmaMinTiles && tiles <= 512u;
     if (batch < 5 && tiles < kMfmaSplitTiles && !q4_0_few) return false;
-    if (batch <= max_register_batch(enc) && bytes < (8ull << 20) && tiles < kMfmaSplitTiles) return false;
+    if (batch <= valu_pass_rows(enc) && bytes < (8ull << 20) && tiles < kMfmaSplitTiles) return false;
     const uint32_t min_tiles = mfma_min_tiles(enc, batch);
     const int mode = enc == ENC_Q4_0   ? mfma_mode<MfmaQ40>(K, tiles, y_bf16, min_tiles)
                    : enc == ENC_Q6_K   ? mfma_mode<MfmaQ6K>(K, tiles, y_bf16, min_tiles)

@@ -20,11 +20,28 @@ hipError_t launch_mlx(const GemvParams& p, uint32_t B, uint32_t oneshot, hipStre
         DMX_ONESHOT(2, 1)
         DMX_ONESHOT(2, 2)
         DMX_ONESHOT(4, 1)
+        DMX_ONESHOT(4, 2)
+        DMX_ONESHOT(4, 4)
+        DMX_ONESHOT(4, 8)
         DMX_ONESHOT(8, 1)
-        // 8 rows of 2 chunks per lane take ~300 registers: 256-thread workgroups only
-        if (B == 8 && oneshot == 2)
-            return launch_oneshot<GemvKernel>(nullptr, mlx_u4_gemv_oneshot_kernel<2, 8, xmode_rows(XM, 8), 256>, p,
-                                              lds, st);
+        DMX_ONESHOT(8, 2)
+        DMX_ONESHOT(8, 4)
+        DMX_ONESHOT(8, 8)
+#define DMX_ONESHOT_SPLIT(b, c)                                                                            \
+    if (B == b && oneshot == (kOneshotSplit | c))                                                          \
+        return launch_oneshot(mlx_u4_gemv_oneshot_kernel<c, b, xmode_rows(XM, b), 512, 4>,                  \
+                              mlx_u4_gemv_oneshot_kernel<c, b, xmode_rows(XM, b), 256, 4>, p, lds, st, 4u);
+#define DMX_ONESHOT_WIDE(c)                                                                                \
+    if (B == 4 && oneshot == (kOneshotWide | c))                                                           \
+        return launch_oneshot_wide(mlx_u4_gemv_oneshot_kernel<c, 4, xmode_rows(XM, 4), 1024, 4>, p, lds, st);
+        DMX_ONESHOT_SPLIT(4, 1)
+        DMX_ONESHOT_SPLIT(4, 2)
+        DMX_ONESHOT_SPLIT(8, 1)
+        DMX_ONESHOT_SPLIT(8, 2)
+        DMX_ONESHOT_WIDE(4)
+        DMX_ONESHOT_WIDE(8)
+#undef DMX_ONESHOT_WIDE
+#undef DMX_ONESHOT_SPLIT
 #undef DMX_ONESHOT
         return hipErrorInvalidValue;
     }

@@ -150,7 +150,7 @@ __device__ __forceinline__ float stream_chunk(const typename E::Chunk& c, const 
     for (int t = 0; t < E::NT; t++) {
         uint32_t pr[E::PPT], xv[E::PPT];
         E::pairs(c, t, pr);
-        load_xpairs<E>(xq, 0u, t, xv);
+        load_xpairs<E>(xq, t, xv);
 #pragma unroll
         for (int h = 0; h < E::PPT; h++) {
             float& a = acc[E::grp(t, h)];

@@ -69,12 +69,17 @@ __host__ __device__ constexpr uint32_t xtile_chunk_bytes(uint32_t enc) {
          : (enc == ENC_Q8_0 || enc == ENC_Q4_0 || enc == ENC_IQ4_XS) ? 20u * 4u + 2u * 4u  // 16 + pad, (-C, s)
          : 20u * 4u + 4u * 4u;                                            // Q4_1, MLX: (-C, s, s.Σx, 0)
 }
+constexpr uint32_t kXRowSkew = 16;  // bytes between the rows of a tile of 4 or 8
 __host__ __device__ constexpr uint64_t xtile_bytes(uint32_t enc, uint32_t B, uint32_t K) {
-    return (uint64_t)B * (K / xtile_chunk_weights(enc)) * xtile_chunk_bytes(enc);
+    return (uint64_t)B * ((K / xtile_chunk_weights(enc)) * xtile_chunk_bytes(enc) + (B >= 4 ? kXRowSkew : 0u));
 }
 // Widest activation batch one GEMV launch holds in registers (wider batches
-// run as several launches): 8 rows, 4 for the 64-weight chunks.
-__host__ __device__ constexpr uint32_t max_register_batch(uint32_t enc) { return wide_chunks(enc) ? 4u : 8u; }
+// run as several launches).
+__host__ __device__ constexpr uint32_t max_register_batch(uint32_t) { return 8u; }
+// Latency mode with four waves per row block (with the chunks per lane in the low bits).
+// kOneshotWide: in workgroups of 1024 threads.
+constexpr uint32_t kOneshotSplit = 0x100u, kOneshotWide = 0x200u;
+constexpr uint32_t kSplitSums = 2048u;  // LDS of their sums besides the activation tile, at most
 // LDS of one gfx950 workgroup.
 constexpr uint32_t kLdsBytes = 160u * 1024u;
 
