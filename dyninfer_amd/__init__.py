@@ -22,6 +22,7 @@ from __future__ import annotations
 import ctypes
 import json
 import os
+import struct
 from dataclasses import dataclass
 from typing import Optional, Sequence
 
@@ -79,6 +80,8 @@ class _QWeightC(ctypes.Structure):
         ("data_bytes", ctypes.c_uint64), ("scales_bytes", ctypes.c_uint64), ("biases_bytes", ctypes.c_uint64),
     ]
 
+
+_pack_qweight = struct.Struct("@2I5Q2I3Q").pack  # _QWeightC's layout
 
 _lib: Optional[ctypes.CDLL] = None
 
@@ -145,6 +148,13 @@ def library() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    # the calls of every step: the weights as packed bytes (QWeight.pack), see Context
+    for name in ("qlinear_multi", "prefill_workspace_bytes", "embedding"):
+        fn = lib["dyninfer_mi355x_" + name]
+        res, args = sig["dyninfer_mi355x_" + name]
+        fn.restype = res
+        fn.argtypes = [P if a is W else a for a in args]
+        setattr(lib, "packed_" + name, fn)
     _lib = lib
     return lib
 
@@ -173,11 +183,15 @@ def _ptr(t) -> Optional[int]:
     return t.data_ptr() if hasattr(t, "data_ptr") else int(t)
 
 
-def _nbytes(t) -> Optional[int]:
-    """Byte length of a tensor (None for a raw address)."""
-    if t is None or not hasattr(t, "data_ptr"):
-        return None
-    return t.numel() * t.element_size()
+def _span(t, nbytes: Optional[int]):
+    """(address, byte length) of a tensor or raw address; None: a length for the encoding to tell."""
+    if t is None:
+        return 0, nbytes
+    try:
+        p = t.data_ptr()
+    except AttributeError:
+        return int(t), nbytes
+    return p, t.numel() * t.element_size() if nbytes is None else nbytes
 
 
 @dataclass
@@ -212,12 +226,26 @@ class QWeight:
         g = self.rows * (self.cols // self.group_size) * es if self.group_size else 0
         return self.rows * self.cols // 2, g, g
 
+    def _fields(self):
+        """The C struct's values in order."""
+        d, dn = _span(self.data, self.data_bytes)
+        s, sn = _span(self.scales, self.scales_bytes)
+        b, bn = _span(self.biases, self.biases_bytes)
+        if dn is None or sn is None or bn is None:
+            ed, es, eb = self._expected()
+            dn, sn, bn = ed if dn is None else dn, es if sn is None else sn, eb if bn is None else bn
+        return (self.encoding, self.group_size, self.rows, self.cols, d, s, b, self.scale_dtype, 0, dn, sn, bn)
+
     def c(self) -> _QWeightC:
-        ed, es, eb = self._expected()
-        pick = lambda given, t, exp: given if given is not None else (_nbytes(t) if _nbytes(t) is not None else exp)
-        return _QWeightC(self.encoding, self.group_size, self.rows, self.cols, _ptr(self.data), _ptr(self.scales),
-                         _ptr(self.biases), self.scale_dtype, 0, pick(self.data_bytes, self.data, ed),
-                         pick(self.scales_bytes, self.scales, es), pick(self.biases_bytes, self.biases, eb))
+        return _QWeightC(*self._fields())
+
+    def pack(self) -> bytes:
+        """The C struct's bytes."""
+        v = self._fields()
+        try:
+            return _pack_qweight(*v)
+        except struct.error:  # out of a field's range: wraps as in C, for the library to refuse
+            return bytes(_QWeightC(*v))
 
     @property
     def nbytes(self) -> int:
@@ -225,15 +253,18 @@ class QWeight:
         return weight_bytes(self.encoding, self.rows, self.cols, self.group_size or 64, sb)
 
 
+_DTYPE_CODES: dict = {}  # torch dtype -> code, filled on first use (torch is imported late)
+
+
 def _dtype_code(t) -> int:
+    code = _DTYPE_CODES.get(t.dtype)
+    if code is not None:
+        return code
     import torch
-    if t.dtype == torch.float32:
-        return DTYPE_F32
-    if t.dtype == torch.bfloat16:
-        return DTYPE_BF16
-    if t.dtype == torch.float16:
-        return DTYPE_F16
-    raise TypeError(f"unsupported dtype {t.dtype}")
+    _DTYPE_CODES.update({torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16})
+    if t.dtype not in _DTYPE_CODES:
+        raise TypeError(f"unsupported dtype {t.dtype}")
+    return _DTYPE_CODES[t.dtype]
 
 
 def supports(w: QWeight, rows: int, x_dtype: int = DTYPE_F32, y_dtype: int = DTYPE_F32) -> bool:
@@ -247,9 +278,14 @@ def prefill_workspace_bytes(ws: Sequence[QWeight], rows: int, x_dtype: int = DTY
     and dtypes (dyninfer_mi355x_prefill_workspace_bytes): required by a call that runs the
     prefill GEMM, optional for a decode call on the MFMA GEMV (which then stages its
     activations once per call), 0 for every other call."""
-    arr = (_QWeightC * len(ws))(*[w.c() for w in ws])
+    return _workspace_bytes(b"".join([w.pack() for w in ws]), len(ws), rows, x_dtype, y_dtype)
+
+
+def _workspace_bytes(packed: bytes, count: int, rows: int, x_dtype: int, y_dtype: int) -> int:
     n = ctypes.c_uint64(0)
-    _check(library().dyninfer_mi355x_prefill_workspace_bytes(arr, len(ws), rows, x_dtype, y_dtype, ctypes.byref(n)))
+    rc = library().packed_prefill_workspace_bytes(packed, count, rows, x_dtype, y_dtype, ctypes.byref(n))
+    if rc:
+        _check(rc)
     return n.value
 
 
@@ -281,25 +317,30 @@ class Context:
         except Exception:
             pass
 
+    # Host time of a call (us; one Q4_0 3072 x 1024 row, three weights of 512 rows, a
+    # gather of 512 rows): 12.2, 20.9, 8.2 -> 7.4, 10.8, 5.0.  The C entry takes 3.8, 6.4 and 3.3
+    # of it, mostly the launches.  Weights go as packed bytes, built once per call; a
+    # caller's workspace goes to the library as it is (it sizes the call itself and
+    # leaves a workspace alone that the call has no use for).
     @staticmethod
     def _stream(stream) -> Optional[int]:
         if stream is None:
             import torch
-            return torch.cuda.current_stream().cuda_stream
+            return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
         return stream if isinstance(stream, int) else stream.cuda_stream
 
-    def _workspace(self, ws, x, rows: int, ydt: int, stream, workspace):
+    def _workspace(self, packed: bytes, count: int, x, rows: int, xdt: int, ydt: int, stream, workspace):
         """(pointer, bytes, keep-alive) of the call's device workspace: the caller's
         ``workspace`` tensor, or a new torch allocation of the size the library asks
         for (torch's caching allocator, tied to the launch stream), or none (also when
         ``workspace`` is False: a decode call then runs without its optional one)."""
-        import torch
         if workspace is False:
             return None, 0, None
-        need = prefill_workspace_bytes(ws, rows, _dtype_code(x), ydt)
-        if need == 0:
-            return None, 0, None
         if workspace is None:
+            need = _workspace_bytes(packed, count, rows, xdt, ydt)
+            if need == 0:
+                return None, 0, None
+            import torch
             workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
             if stream is not None:
                 st = stream if isinstance(stream, torch.cuda.Stream) else torch.cuda.ExternalStream(int(stream))
@@ -311,15 +352,7 @@ class Context:
         workspace: a device tensor of at least prefill_workspace_bytes([w], rows, …)
         bytes (one is allocated through torch when omitted and that size is not 0), or
         False for none (decode calls only)."""
-        import torch
-        rows = x.shape[0] if x.dim() == 2 else 1
-        if y is None:
-            y = torch.empty((rows, w.rows), dtype=y_dtype or torch.float32, device=x.device)
-        wp, wn, _keep = self._workspace([w], x, rows, _dtype_code(y), stream, workspace)
-        wc = w.c()
-        _check(self._lib.dyninfer_mi355x_qlinear(self._h, ctypes.byref(wc), x.data_ptr(), _dtype_code(x), rows,
-                                                 y.data_ptr(), _dtype_code(y), wp, wn, self._stream(stream)))
-        return y
+        return self.qlinear_multi((w,), x, None if y is None else (y,), y_dtype, stream, workspace=workspace)[0]
 
     def qlinear_multi(self, ws: Sequence[QWeight], x, ys=None, y_dtype=None, stream=None, noalloc=False,
                       workspace=None):
@@ -331,15 +364,17 @@ class Context:
         rows = x.shape[0] if x.dim() == 2 else 1
         if ys is None:
             ys = [torch.empty((rows, w.rows), dtype=y_dtype or torch.float32, device=x.device) for w in ws]
-        arr = (_QWeightC * len(ws))(*[w.c() for w in ws])
-        yp = (ctypes.c_void_p * len(ws))(*[y.data_ptr() for y in ys])
+        n, xdt, ydt = len(ws), _dtype_code(x), _dtype_code(ys[0])
+        yp = (ctypes.c_void_p * n)(*[y.data_ptr() for y in ys])
         if noalloc:
-            _check(self._lib.dyninfer_mi355x_qlinear_multi_noalloc(self._h, arr, len(ws), x.data_ptr(), _dtype_code(x),
-                                                                   rows, yp, _dtype_code(ys[0]), self._stream(stream)))
+            arr = (_QWeightC * n)(*[w.c() for w in ws])
+            _check(self._lib.dyninfer_mi355x_qlinear_multi_noalloc(self._h, arr, n, x.data_ptr(), xdt, rows, yp, ydt,
+                                                                   self._stream(stream)))
             return ys
-        wp, wn, _keep = self._workspace(ws, x, rows, _dtype_code(ys[0]), stream, workspace)
-        _check(self._lib.dyninfer_mi355x_qlinear_multi(self._h, arr, len(ws), x.data_ptr(), _dtype_code(x), rows, yp,
-                                                       _dtype_code(ys[0]), wp, wn, self._stream(stream)))
+        packed = ws[0].pack() if n == 1 else b"".join([w.pack() for w in ws])
+        wp, wn, _keep = self._workspace(packed, n, x, rows, xdt, ydt, stream, workspace)
+        _check(self._lib.packed_qlinear_multi(self._h, packed, n, x.data_ptr(), xdt, rows, yp, ydt, wp, wn,
+                                              self._stream(stream)))
         return ys
 
     def dequant(self, w: QWeight, out=None, stream=None):
@@ -360,9 +395,8 @@ class Context:
         n = ids.numel()
         if out is None:
             out = torch.empty((n, w.cols), dtype=torch.float32, device=ids.device)
-        wc = w.c()
-        _check(self._lib.dyninfer_mi355x_embedding(self._h, ctypes.byref(wc), ids.data_ptr() if n else None, n,
-                                                   out.data_ptr() if n else None, self._stream(stream)))
+        _check(self._lib.packed_embedding(self._h, w.pack(), ids.data_ptr() if n else None, n,
+                                         out.data_ptr() if n else None, self._stream(stream)))
         return out
 
 
