@@ -215,22 +215,30 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
     uint32_t oneshot = cpl >= 1 && cpl <= max_cpl && rbs1 <= max_rbs ? cpl : 0u;
     if (B >= 4) {
         // 4 and 8 rows, a row block being four rows by sixteen lanes.  Up to 512 row
-        // blocks (1024 at 4 rows from K = 2048) one wave each would leave most SIMDs
-        // idle: four waves share one (us per launch, one wave against four: MLX 1024 x
-        // 3072 at 8 rows 8.8 -> 6.5, Q8_0 10.8 -> 8.6, Q6_K 1024 x 4096 at 4 rows 7.6
-        // -> 5.1, Q4_0 4096 x 4096 at 4 rows 6.5 -> 6.2; but 4096 x 1024 4.1 -> 4.8 and
-        // 4096 x 4096 at 8 rows 9.7 -> 11.9: every workgroup stages the activations).
-        // Where the activations leave one workgroup per CU it has 1024 threads (Q4_0
-        // 4096 x 12288 at 4 rows 17.3 -> 15.0; 64-weight chunks spill there).  One
-        // wave per row block up to 8192 of them at 1..2 chunks per lane (MLX 6144 x
-        // 1024 at 8 rows 5.8 us in the pipeline, 5.3) and 2048 at more (Q4_0 6144 x
-        // 4096 at 4 rows 10.2 against 8.0; Q4_0 24576 x 4096 16.4 against 20.5).
+        // blocks (1024 at 4 rows from K = 2048, two workgroups to a CU) one wave each
+        // would leave most SIMDs idle: four waves share one (us per launch, one wave
+        // against four: MLX 1024 x 3072 at 8 rows 8.8 -> 6.5, Q8_0 10.8 -> 8.6, Q6_K
+        // 1024 x 4096 at 4 rows 7.6 -> 5.1, 2048 x 14336 18.8 -> 14.5, Q4_0 4096 x 4096
+        // 6.5 -> 6.2; but 4096 x 1024 4.1 -> 4.8 and 4096 x 4096 at 8 rows 9.7 -> 11.9:
+        // every workgroup stages the activations).  Where these leave one workgroup per
+        // CU it has four row blocks, all its loads in flight at once (4 rows, the
+        // pipeline against this: Q4_0 4096 x 12288 17.3 -> 14.0, Q4_K 17.2 -> 15.8, Q6_K
+        // 20.3 -> 19.2, Q8_0 -> 20.2, Q4_K 4096 x 8192 13.3 -> 10.9), while the CUs take
+        // all row blocks at once (Q4_K 8192 x 12288, two rounds, 20.0 -> 29.2) and the
+        // chunks fit the registers (Q5_K 4096 x 14336, eight a lane, 24.0 -> 27.0).  One
+        // wave per row block up to 8192 of them at 1..2 chunks per lane (MLX 6144 x 1024
+        // at 8 rows 5.8 us in the pipeline, 5.3) and 2048 at more (Q4_0 6144 x 4096 at 4
+        // rows 10.2 against 8.0; Q4_0 24576 x 4096 16.4 against 20.5).
         const uint64_t tile = xtile_bytes(enc, B, K);
         const uint32_t cps = (nch + 63u) / 64u;  // chunks per lane, four waves per row block
-        if (cps <= 2u && tile + kSplitSums <= lim && (rbs1 <= 512u || (B == 4u && rbs1 <= 1024u && K >= 2048u)))
-            oneshot = kOneshotSplit | cps;
-        else if (!info.wide && B == 4u && rbs1 <= 2048u && tile > kLdsBytes / 2u && tile + kSplitSums <= lim && cps <= 8u)
-            oneshot = kOneshotWide | (cps <= 4u ? 4u : 8u);
+        const uint32_t cpw = info.wide ? (nch + 31u) / 32u : cps;
+        const bool one_per_cu = tile > kLdsBytes / 2u;
+        const uint32_t max_cps = B == 4u ? (info.wide ? 4u : 8u) : 2u;
+        if (tile + kSplitSums <= lim &&
+            ((rbs1 <= 512u && cps <= max_cps) || (B == 4u && rbs1 <= 1024u && K >= 2048u && cps <= 2u && !one_per_cu)))
+            oneshot = kOneshotSplit | (cps <= 2u ? cps : cps <= 4u ? 4u : 8u);
+        else if (B == 4u && rbs1 <= 1024u && one_per_cu && tile + kSplitSums <= lim && cpw <= (info.wide ? 6u : 7u))
+            oneshot = kOneshotWide | (cpw <= 4u ? 4u : cpw <= 6u ? 6u : 7u);
         else if (cpl <= 2u) oneshot = rbs1 <= 8192u ? cpl : 0u;
         else oneshot = rbs1 <= 2048u && cpl <= (info.wide ? 4u : 8u) ? (cpl <= 4u ? 4u : 8u) : 0u;
     }

@@ -33,13 +33,16 @@ hipError_t launch_mlx(const GemvParams& p, uint32_t B, uint32_t oneshot, hipStre
                               mlx_u4_gemv_oneshot_kernel<c, b, xmode_rows(XM, b), 256, 4>, p, lds, st, 4u);
 #define DMX_ONESHOT_WIDE(c)                                                                                \
     if (B == 4 && oneshot == (kOneshotWide | c))                                                           \
-        return launch_oneshot_wide(mlx_u4_gemv_oneshot_kernel<c, 4, xmode_rows(XM, 4), 1024, 4>, p, lds, st);
+        return launch_oneshot_wide(mlx_u4_gemv_oneshot_kernel<c, 4, xmode_rows(XM, 4), 1024, 4>, p, lds, st, 1024);
         DMX_ONESHOT_SPLIT(4, 1)
         DMX_ONESHOT_SPLIT(4, 2)
+        DMX_ONESHOT_SPLIT(4, 4)
+        DMX_ONESHOT_SPLIT(4, 8)
         DMX_ONESHOT_SPLIT(8, 1)
         DMX_ONESHOT_SPLIT(8, 2)
         DMX_ONESHOT_WIDE(4)
-        DMX_ONESHOT_WIDE(8)
+        DMX_ONESHOT_WIDE(6)
+        DMX_ONESHOT_WIDE(7)
 #undef DMX_ONESHOT_WIDE
 #undef DMX_ONESHOT_SPLIT
 #undef DMX_ONESHOT

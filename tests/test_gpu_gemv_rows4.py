@@ -55,8 +55,13 @@ SHAPES = [
     (7, [2051, 64], 1024),        # ... two
     (6, [3001], 1792),            # ... four, some lanes with fewer
     (8, [2077], 3840),            # ... eight of 32 weights
-    (4, [4090], 12288),           # 1024 threads to a workgroup, or the pipeline
+    (4, [4090], 12288),           # four row blocks to a workgroup, one per CU
     (3, [2050], 8448),
+    (4, [2051], 14336),           # ... seven chunks a lane, or the pipeline
+    (4, [1030, 250], 7936),       # ... four
+    (4, [1500], 14336),           # four waves per row block, up to eight chunks a lane
+    (3, [1026], 6144),
+    (4, [8200], 7680),            # one workgroup to a CU, more row blocks than they take at once
     (8, [2100], 5120),            # the pipeline, one workgroup to a CU
     (4, [33001], 256),
     (8, [8197, 8197], 768),
