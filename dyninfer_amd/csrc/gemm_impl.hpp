@@ -934,19 +934,19 @@ void gemm_kernel(const GemmArgs a) {
     // slice's 4·TM·WM per chunk (f = 4·i + t: row block i, k step t).
     constexpr bool XR = G::XR;
     constexpr uint32_t NX = XR ? TM : G::kDmaX;
-    Src xbase;
-    xbase.set(a.xh);
+    Src xbase;  // the tile's first row block: the rows rounded up to 32 may pass 4 GiB in all
+    xbase.set(a.xh + (size_t)mb0 * ksteps * 512u);
     uint32_t xsrc[NX], xdst[NX];
     if constexpr (XR) {  // row block q's fragments of the slice
 #pragma unroll
         for (uint32_t q = 0; q < NX; q++)
-            xsrc[q] = ((mb0 + q < mbs ? mb0 + q : mbs - 1u) * ksteps + 4u * c0) * 1024u;
+            xsrc[q] = ((mb0 + q < mbs ? q : mbs - 1u - mb0) * ksteps + 4u * c0) * 1024u;
     }
 #pragma unroll
     for (uint32_t q = 0; !XR && q < NX; q++) {
         const uint32_t f = ns + WN * wm + q * (uint32_t)(WN * WM), i = f / 4u, t = f % 4u;
-        const uint32_t mb = mb0 + i < mbs ? mb0 + i : mbs - 1u;  // past M: re-read the last block (never stored)
-        xsrc[q] = (mb * ksteps + 4u * c0 + t) * 1024u;  // rows·K < 2^31: below 4 GiB
+        const uint32_t mb = mb0 + i < mbs ? i : mbs - 1u - mb0;  // past M: re-read the last block (never stored)
+        xsrc[q] = (mb * ksteps + 4u * c0 + t) * 1024u;
         xdst[q] = (ks * 4u * TM * WM + f) * 1024u;
     }
     W win;

@@ -84,3 +84,20 @@ def test_gemm_plans(ctx, kind, m, ns, k):
                                     (300, [20000], 64)])
 def test_gemm_plans_odd_chunks(ctx, kind, m, ns, k):
     check(ctx, kind, m, ns, k)
+
+
+@pytest.mark.parametrize("n", [33, 260])
+def test_gemm_activations_past_4gib(ctx, n):
+    """rows·K just below the limit of 2^31: rounded up to 32 rows the staged activations pass
+    4 GiB, and the last rows' fragments lie beyond a 32-bit offset."""
+    k, tail = 20480, 57
+    m = (2**31 - 1) // k
+    w, wf, _ = weight("q8_0", n, k, seed=5)
+    x = torch.zeros(m, k, dtype=torch.bfloat16, device="cuda")
+    x[-tail:] = torch.from_numpy(oracle.randn(tail * k, seed=6).reshape(tail, k)).cuda().bfloat16()
+    y = ctx.qlinear(w, x)
+    assert not y[:-tail].any()
+    xt = x[-tail:].float().cpu().numpy()
+    y64, absdot = oracle.linear_f64(xt, wf)
+    err = np.abs(y[-tail:].cpu().numpy().astype(np.float64) - y64)
+    assert (err <= (2.0 ** -10 + 2e-5) * absdot).all(), float((err / absdot).max())
