@@ -469,7 +469,8 @@ struct WinQ6K {
 // word = k offset i, fixture.rs:307-311): a row's chunk is 8 words (32 bytes,
 // 4-byte-aligned rows of K/2 bytes) copied as two 16-byte pieces, plus, per
 // row, the dwords holding the scale and the bias of the chunk's two 32-k
-// halves (the same group unless group = 32).  Lane l decodes row 32j + l % 32
+// halves (always the same group only where 64 divides the group size: a chunk of
+// groups of 96 may start in one group and end in the next).  Lane l decodes row 32j + l % 32
 // of each N-block j, words 4h .. 4h+3 (h = l / 32): k step t takes word
 // 4h + t, nibbles (0,4) (1,5) (2,6) (3,7) as packed pairs (XFRAG_WORD), code q
 // exact in f16 and w = RNE_f16(q·s + b) by one packed fma, s and b taken to
@@ -481,7 +482,7 @@ struct WinMlx {
     static constexpr uint32_t kMine = (kPieces + PARTS - 1u) / PARTS;
     static constexpr uint32_t kAuxQ = (kRows + 63u) / 64u;       // 4-byte copies per scale or bias array
     // the scales and biases of one group (PARTS 2: one wave copies the scales, the
-    // other the biases); a second copy of each, not counted, with groups of 32
+    // other the biases); a second copy of each, not counted, where halves differ
     static constexpr uint32_t kCopies = kMine + 2u / PARTS * kAuxQ;
     static constexpr uint32_t kAuxOff = kPieces * 1024u;         // the aux dwords after every row's pieces
     static constexpr uint32_t kAuxPitch = 256u * kAuxQ;          // bytes per aux array: s0, s1, b0, b1
@@ -494,13 +495,13 @@ struct WinMlx {
     uint32_t src[kMine], dst[kMine];         // copy lane's piece of the slice's first chunk, from base; its place
     uint32_t srow[kAuxQ], brow[kAuxQ];       // copy lane's row of scales and biases, from sbase and bbase
     uint32_t ssh[NB], bsh[NB];               // this lane's rows' scale and bias row starts mod 4 (per N-block j)
-    uint32_t c0, es, gmagic, m32, m16, lane, mine, g32;  // (m32, m16: all ones for f32, f16 scales; g32: groups of 32)
+    uint32_t c0, es, gmagic, m32, m16, lane, mine, two;  // (m32, m16: all ones for f32, f16 scales; two: halves' groups differ)
 
     __device__ void init(const GemmArgs& a, const GemmProb& pr, uint32_t n0, uint32_t lane_, uint32_t c0_, uint32_t part) {
         lane = lane_;
         c0 = c0_;
         mine = part;
-        g32 = a.group < 64u ? 1u : 0u;
+        two = a.group % 64u ? 1u : 0u;
         gmagic = a.gmagic;
         m32 = a.sdtype == DT_F32 ? ~0u : 0u;
         m16 = a.sdtype == DT_F16 ? ~0u : 0u;
@@ -543,7 +544,7 @@ struct WinMlx {
                     bbase.dma4((brow[q] + o) & ~3u, 0u, win + kAuxOff + kAuxPitch * (2u + hh) + 256u * q);
             }
         };
-        if (g32) aux(1);  // more copies than the waits count: they wait for older ones than they must
+        if (two) aux(1);  // more copies than the waits count: they wait for older ones than they must
 #pragma unroll
         for (uint32_t q = 0; q < kMine; q++) base.dma16(src[q], c * 32u, win + dst[q]);
         aux(0);
@@ -559,8 +560,8 @@ struct WinMlx {
             o[1] = q.y;
             o[2] = q.z;
             o[3] = q.w;
-            o[4] = *reinterpret_cast<const uint32_t*>(win + kAuxOff + kAuxPitch * (h * g32) + 4u * r);
-            o[5] = *reinterpret_cast<const uint32_t*>(win + kAuxOff + kAuxPitch * (2u + h * g32) + 4u * r);
+            o[4] = *reinterpret_cast<const uint32_t*>(win + kAuxOff + kAuxPitch * (h * two) + 4u * r);
+            o[5] = *reinterpret_cast<const uint32_t*>(win + kAuxOff + kAuxPitch * (2u + h * two) + 4u * r);
         }
     }
     __device__ Scale scale(uint32_t c, int j, const uint32_t* r) const {

@@ -101,3 +101,45 @@ def test_gemm_activations_past_4gib(ctx, n):
     y64, absdot = oracle.linear_f64(xt, wf)
     err = np.abs(y[-tail:].cpu().numpy().astype(np.float64) - y64)
     assert (err <= (2.0 ** -10 + 2e-5) * absdot).all(), float((err / absdot).max())
+
+
+def _shifted(a, off):
+    """a on the device, its first byte `off` bytes past a 4-byte boundary."""
+    t = torch.zeros(a.nbytes + 4, dtype=torch.uint8, device="cuda")
+    t[off:off + a.nbytes] = torch.from_numpy(a.view(np.uint8).reshape(-1)).cuda()
+    return t[off:off + a.nbytes]
+
+
+@pytest.mark.parametrize("sdtype,off", [(oracle.D_BF16, 0), (oracle.D_BF16, 2), (oracle.D_F16, 2), (oracle.D_F32, 0)])
+@pytest.mark.parametrize("group,m,ns,k", [
+    (96, 40, [97], 192),      # 2 2 1 4 1
+    (96, 41, [97, 60], 384),  # 1 1 4 1 1
+    (160, 45, [131], 960),    # 1 1 8 1 1
+    (96, 45, [131], 960),
+    (160, 20, [1000], 320),   # fewer rows than a row block
+    (96, 257, [14002], 192),  # 4 2 1 2 2: one of the two waves of a window copies the scales, one the biases
+    (160, 260, [14002], 320),
+])
+def test_gemm_mlx_groups_across_chunks(ctx, sdtype, off, group, m, ns, k):
+    """Group sizes that are multiples of 32 and not of 64: a group may end in the middle of a
+    64-k chunk, whose halves then take scales and biases of two groups.
+
+    f32 scales and biases are rounded to f16 first: 2^-11 (|q s| + |b|) |x| besides, and
+    |q s| <= |w| + |b|."""
+    ws, refs = [], []
+    for n in ns:
+        packed, sc, bi = oracle.synth_mlx_u4(n, k, group, sdtype, seed=n + k + group)
+        ws.append(d.QWeight(d.ENC_MLX_U4, n, k, torch.from_numpy(packed).cuda(), _shifted(sc, off), _shifted(bi, off),
+                            group, sdtype))
+        wf = oracle.dequant_mlx_u4(packed, sc, bi, sdtype, n, k, group)
+        b = np.repeat(np.abs(bi.astype(np.float64)).reshape(n, -1), group, axis=1) if sdtype == oracle.D_F32 else None
+        refs.append((wf, b))
+    x = oracle.randn(m * k, seed=m + k).reshape(m, k)
+    ys = ctx.qlinear_multi(ws, torch.from_numpy(x).cuda())
+    for y, (wf, b) in zip(ys, refs):
+        y64, absdot = oracle.linear_f64(x, wf)
+        bound = (2.0 ** -10 + 2e-5) * absdot
+        if b is not None:
+            bound = bound + 2.0 ** -11 * (absdot + 2.0 * (np.abs(x).astype(np.float64) @ b.T))
+        err = np.abs(y.cpu().numpy().astype(np.float64) - y64)
+        assert (err <= bound).all(), float((err / absdot).max())
