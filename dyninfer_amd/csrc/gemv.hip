@@ -111,28 +111,6 @@ hipError_t launch(uint32_t enc, const GemvParams& p, uint32_t B, uint32_t onesho
 
 }  // namespace
 
-// Whether a launch of 3..8 rows that the 16-row MFMA GEMV could serve runs the 4x4
-// MFMA kernels instead (chunk_dot4): 3..4 rows, all but Q6_K from 4096 tiles of 16
-// rows (151936 x 4096: 112 us on the 16-row path against 117); 5..8 rows, launches
-// below 8 MB and 1024 tiles (Q6_K 1024 x 4096 at 8 rows 9.4 -> 7.4 us; Q4_K 4096 x
-// 4096, 9.4 MB, 9.8 us on the 16-row path against 10.9).
-static bool gemv_prefers_4x4(uint32_t enc, const GemvProblem* probs, int nprob, uint32_t batch, uint32_t K) {
-    if (batch > 8u) return false;
-    uint64_t tiles = 0, rows = 0;
-    for (int i = 0; i < nprob; i++) {
-        tiles += (probs[i].n + 15u) / 16u;
-        rows += probs[i].n;
-    }
-    if (batch <= 4u) return enc != ENC_Q6_K || tiles < 4096u;
-    const uint64_t row = enc == ENC_Q4_0   ? K / 32u * 18u
-                         : enc == ENC_Q6_K ? K / 256u * 210u
-                         : enc == ENC_Q4_K ? K / 256u * 144u
-                         : enc == ENC_Q5_K ? K / 256u * 176u
-                         : enc == ENC_IQ4_XS ? K / 256u * 136u
-                                             : K / 2u;
-    return rows * row < (8ull << 20) && tiles < 1024u;
-}
-
 uint64_t gemv_workspace_bytes(uint32_t enc, const GemvProblem* probs, int nprob, uint32_t batch, uint32_t K,
                               bool y_bf16, uint32_t group) {
     if (nprob < 1 || nprob > kMaxProblems) return 0;
@@ -147,12 +125,11 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
         return hipErrorInvalidValue;
     // 9..16 activation rows, and 3..8 on large launches: every weight decoded once for
     // all rows, on 16-row MFMAs
-    const bool m4 = gemv_prefers_4x4(enc, probs, nprob, batch, K);
-    if (!m4 && gemv_mfma_applies(enc, probs, nprob, batch, K, y_bf16, group))
+    if (gemv_mfma_applies(enc, probs, nprob, batch, K, y_bf16, group))
         return gemv_mfma_launch(enc, probs, nprob, K, x, x_bf16, batch, y_bf16, group, sdtype, work, work_bytes,
                                 stream);
     // bf16 outputs and K in several segments: on MFMA when the workspace holds f32 accumulators
-    if (!m4 && y_bf16 && work) {
+    if (y_bf16 && work) {
         const uint64_t need = gemv_mfma_bf16_acc_bytes(enc, probs, nprob, batch, K, group);
         if (need && work_bytes >= need)
             return gemv_mfma_launch_bf16_acc(enc, probs, nprob, K, x, x_bf16, batch, group, sdtype, work, work_bytes,

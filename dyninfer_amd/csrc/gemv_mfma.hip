@@ -1180,18 +1180,14 @@ hipError_t launch_mode(MfmaParams p, uint32_t units, bool y_bf16, uint8_t* pre, 
 template <class M>
 int mfma_mode(uint32_t K, uint32_t tiles, bool y_bf16, uint32_t min_tiles);
 
-// Up to these rows a launch has another single-pass kernel, which small launches keep.
-uint32_t valu_pass_rows(uint32_t enc) { return wide_chunks(enc) ? 4u : 8u; }
-
-uint32_t mfma_min_tiles(uint32_t enc, uint32_t batch) {
-    return batch > valu_pass_rows(enc) ? kMfmaMinTilesTwoPasses : kMfmaMinTiles;
-}
+// (up to 8 rows the other kernels take one pass)
+uint32_t mfma_min_tiles(uint32_t batch) { return batch > 8u ? kMfmaMinTilesTwoPasses : kMfmaMinTiles; }
 
 template <class M>
 hipError_t launch_mfma(uint32_t enc, const GemvProblem* probs, int nprob, uint32_t K, const void* x, bool x_bf16,
                        uint32_t batch, bool y_bf16, uint32_t group, uint32_t sdtype, void* work, uint64_t work_bytes,
                        hipStream_t st) {
-    const uint32_t min_tiles = mfma_min_tiles(enc, batch);
+    const uint32_t min_tiles = mfma_min_tiles(batch);
     MfmaParams p = {};
     uint32_t tiles = 0;
     for (int i = 0; i < kMaxProblems; i++) {
@@ -1249,35 +1245,22 @@ bool gemv_mfma_applies(uint32_t enc, const GemvProblem* probs, int nprob, uint32
         tiles += (probs[i].n + 15u) / 16u;
         rows += probs[i].n;
     }
-    // The MFMA path's fixed costs (staging every activation row per
-    // workgroup, a wave's first products) outweigh the VALU GEMV's per-row
-    // work on small launches that the VALU GEMV serves in one register pass:
-    // it takes launches with more rows than one pass holds, launches of at
-    // least 8 MB of weights, or at least kMfmaSplitTiles tiles (measured at
-    // the Qwen3-0.6B MLX shapes: 1-4 MB launches take ~13 us on MFMA against
-    // 7-9 us on VALU at 5-8 rows, 13-15 against 14-18 us at 16 rows).
-    // At 3-4 rows only the largest launches gain (8B lm_head at 4 rows: 114 us on MFMA against 181 us;
-    // at 2 rows both take ~111 us).
     const uint64_t bytes = rows * (enc == ENC_Q4_0   ? K / 32u * 18u
                                    : enc == ENC_Q6_K ? K / 256u * 210u
                                    : enc == ENC_Q4_K ? K / 256u * 144u
                                    : enc == ENC_Q5_K ? K / 256u * 176u
                                    : enc == ENC_IQ4_XS ? K / 256u * 136u
                                                      : K / 2u);
-    // (Launches of 3..8 rows that the 4x4 MFMA kernels run faster are taken out before,
-    // gemv.hip gemv_prefers_4x4; the figures here and below are against v_dot2 kernels.)
-    // At 3-4 rows the VALU GEMV's per-row dot products are cheap enough that
-    // only the largest launches gain, and Q4_0 (the cheapest MFMA decode) with
-    // K = 4096 on 384-512 tiles: per launch at 4 rows, the 8B q/k/v (384 tiles)
-    // 10.58 -> 9.82 us, 8192 x 4096 11.6 -> 11.3; o_proj (256 tiles) 7.5 -> 7.9,
-    // the Q6_K down_proj 17.9 -> 20.2 and the Q4_K q/k 10.0 -> 10.5 stay on
-    // VALU, and so do other Q4_0 shapes (10240 x 4096 12.9 -> 14.5, 14336 x
-    // 4096 17.0 -> 17.5, 6144 x 5120 14.3 -> 17.6, 13824 x 5120 23.0 -> 29.1,
-    // 6144 x 8192 15.8 -> 19.6 on MFMA).
-    const bool q4_0_few = enc == ENC_Q4_0 && K == 4096u && tiles >= kMfmaMinTiles && tiles <= 512u;
-    if (batch < 5 && tiles < kMfmaSplitTiles && !q4_0_few) return false;
-    if (batch <= valu_pass_rows(enc) && bytes < (8ull << 20) && tiles < kMfmaSplitTiles) return false;
-    const uint32_t min_tiles = mfma_min_tiles(enc, batch);
+    // 3..8 rows have another single-pass kernel (4x4 MFMAs, gemv_kernels.hpp chunk_dot4),
+    // without this one's fixed costs (a workgroup stages every activation row before its
+    // first products).  3..4 rows: it takes all but Q6_K from 4096 tiles of 16 rows
+    // (151936 x 4096: 112 us here against 117).  5..8 rows: launches below 8 MB and 1024
+    // tiles (Q6_K 1024 x 4096 at 8 rows 9.4 us here, 7.4 there; Q4_K 4096 x 4096, 9.4 MB,
+    // 9.8 us here against 10.9).
+    if (batch <= 4u ? enc != ENC_Q6_K || tiles < 4096u
+                    : batch <= 8u && bytes < (8ull << 20) && tiles < kMfmaSplitTiles)
+        return false;
+    const uint32_t min_tiles = mfma_min_tiles(batch);
     const int mode = enc == ENC_Q4_0   ? mfma_mode<MfmaQ40>(K, tiles, y_bf16, min_tiles)
                    : enc == ENC_Q6_K   ? mfma_mode<MfmaQ6K>(K, tiles, y_bf16, min_tiles)
                    : enc == ENC_Q4_K   ? mfma_mode<MfmaQ4K>(K, tiles, y_bf16, min_tiles)
@@ -1293,7 +1276,7 @@ uint64_t gemv_mfma_workspace_bytes(uint32_t enc, const GemvProblem* probs, int n
         return y_bf16 ? gemv_mfma_bf16_acc_bytes(enc, probs, nprob, batch, K, group) : 0;
     uint32_t tiles = 0;
     for (int i = 0; i < nprob; i++) tiles += (probs[i].n + 15u) / 16u;
-    const uint32_t min_tiles = mfma_min_tiles(enc, batch);
+    const uint32_t min_tiles = mfma_min_tiles(batch);
     auto size = [&](auto pol) -> uint64_t {
         using M = decltype(pol);
         if (!mfma_prestages<M>(K, batch, mfma_mode<M>(K, tiles, y_bf16, min_tiles))) return 0;

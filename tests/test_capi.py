@@ -187,6 +187,16 @@ def test_prefill_workspace_bytes_follows_the_routing(enc, k):
         assert d.prefill_workspace_bytes(ws[:1], rows) == _ws_bytes(rows, k)
 
 
+@pytest.mark.parametrize("enc", [d.ENC_Q4_0, d.ENC_Q6_K, d.ENC_Q4_K, d.ENC_Q5_K, d.ENC_IQ4_XS])
+@pytest.mark.parametrize("rows,n,k", [(3, 24576, 5120), (4, 16400, 8192), (4, 6144, 12288), (5, 700, 5120), (8, 256, 6144)])
+@pytest.mark.parametrize("y_dtype", [d.DTYPE_F32, d.DTYPE_BF16])
+def test_decode_workspace_is_zero_where_none_is_used(enc, rows, n, k, y_dtype):
+    """Launches of 3..8 rows on the 4x4 MFMA kernels stage their own activations, also where
+    the 16-row MFMA GEMV would take K in several segments."""
+    assert d.prefill_workspace_bytes([w(enc, n, k)], rows, d.DTYPE_F32, y_dtype) == 0
+    assert d.prefill_workspace_bytes([w(enc, 6144, k)], 16, d.DTYPE_F32, y_dtype) >= _decode_ws_bytes(enc, k)
+
+
 def test_prefill_workspace_bytes_validates_like_the_call():
     lib = d.library()
     arr = (d._QWeightC * 2)(w(d.ENC_Q4_0, 64, 1024).c(), w(d.ENC_Q4_0, 64, 512).c())

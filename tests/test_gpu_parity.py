@@ -231,10 +231,10 @@ def test_gemv_mfma(ctx, gtype, n, k, batch, ybf16, off):
 # are identical (K segments add atomically, in either order: within 1e-6 of
 # Σ|w||x|).  The workspace starts as 0xFF bytes (NaN in f16 and f32), so
 # activation rows the prep kernel leaves unstaged (past the batch rounded up
-# to 4, 8 or 16) must not reach a stored output.  3 rows take the MFMA GEMV
-# on >= 1024 tiles only: 1025 tiles, the oracle on the first 2048 rows.
+# to 4, 8 or 16) must not reach a stored output.  5..8 rows take the MFMA GEMV
+# from 8 MB or 1024 tiles: 1025 tiles, the oracle on the first 2048 rows.
 PRESTAGE_CASES = [c for c in MFMA_CASES if c[2] >= 2048 and (c[3] > 8 or c[2] > 4096)] + [
-    (oracle.Q4_0, 16400, 8192, 3, False, 0), (oracle.Q4_K, 6144, 4096, 16, False, 0),
+    (oracle.Q4_0, 16400, 8192, 5, False, 0), (oracle.Q4_K, 6144, 4096, 16, False, 0),
     (oracle.Q5_K, 4096, 12288, 9, False, 0), (oracle.IQ4_XS, 6144, 2048, 12, True, 0),
     # split mode, 16 tasks per segment: each wave's staged operands in registers
     (oracle.Q4_0, 4096, 4096, 16, False, 0), (oracle.Q4_K, 4096, 12288, 16, False, 0),
