@@ -1251,15 +1251,25 @@ bool gemv_mfma_applies(uint32_t enc, const GemvProblem* probs, int nprob, uint32
                                    : enc == ENC_Q5_K ? K / 256u * 176u
                                    : enc == ENC_IQ4_XS ? K / 256u * 136u
                                                      : K / 2u);
-    // 3..8 rows have another single-pass kernel (4x4 MFMAs, gemv_kernels.hpp chunk_dot4),
-    // without this one's fixed costs (a workgroup stages every activation row before its
-    // first products).  3..4 rows: it takes all but Q6_K from 4096 tiles of 16 rows
-    // (151936 x 4096: 112 us here against 117).  5..8 rows: launches below 8 MB and 1024
-    // tiles (Q6_K 1024 x 4096 at 8 rows 9.4 us here, 7.4 there; Q4_K 4096 x 4096, 9.4 MB,
-    // 9.8 us here against 10.9).
-    if (batch <= 4u ? enc != ENC_Q6_K || tiles < 4096u
-                    : batch <= 8u && bytes < (8ull << 20) && tiles < kMfmaSplitTiles)
-        return false;
+    // 3..8 rows have another kernel (4x4 MFMAs, gemv_kernels.hpp chunk_dot4), of one pass
+    // while its activation tile of 4 or 8 rows fits LDS (K up to ~14.8k or ~7.4k) and without
+    // this one's fixed costs (a workgroup stages every activation row before its first
+    // products).  One pass: 3..4 rows go there, all but Q6_K from 4096 tiles of 16 rows
+    // (151936 x 4096: 112 us here against 117), and 5..8 rows below 8 MB and 1024 tiles
+    // (Q6_K 1024 x 4096 at 8 rows 9.4 us here, 7.4 there; Q4_K 4096 x 4096, 9.4 MB, 9.8 us
+    // here against 10.9).  Longer K, each pass reading all weights: 3..4 rows stay here from
+    // 1024 tiles (4 rows, here against there: Q6_K 16384 x 16384 70 us, 93, IQ4_XS 74, 89,
+    // Q4_0 24576 x 16384 0.85 of its time), MLX and three rows of Q4_K from 1536 (16384 x
+    // 16384 1.04 and 1.07 of theirs, 24576 0.96 and 0.95); 5..8 rows of 64-weight chunks from
+    // seven rows or K = 8192 (768 x 12288 at 8 rows: Q4_K 13.6 us, 23.8, Q6_K 15.1, 21.4; K =
+    // 7680 at 5 rows, passes of four and one, 1.08 to 1.22 of their time).
+    const bool one_pass = xtile_bytes(enc, batch <= 4u ? 4u : 8u, K) <= kLdsBytes;
+    if (batch <= 4u) {
+        const uint32_t long_k = enc == ENC_MLX_U4 || (enc == ENC_Q4_K && batch == 3u) ? 1536u : kMfmaSplitTiles;
+        if (one_pass ? enc != ENC_Q6_K || tiles < 4096u : tiles < long_k) return false;
+    } else if (batch <= 8u && bytes < (8ull << 20) && tiles < kMfmaSplitTiles) {
+        if (!wide_chunks(enc) || one_pass || (batch < 7u && K < 8192u)) return false;
+    }
     const uint32_t min_tiles = mfma_min_tiles(batch);
     const int mode = enc == ENC_Q4_0   ? mfma_mode<MfmaQ40>(K, tiles, y_bf16, min_tiles)
                    : enc == ENC_Q6_K   ? mfma_mode<MfmaQ6K>(K, tiles, y_bf16, min_tiles)

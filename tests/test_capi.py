@@ -197,6 +197,16 @@ def test_decode_workspace_is_zero_where_none_is_used(enc, rows, n, k, y_dtype):
     assert d.prefill_workspace_bytes([w(enc, 6144, k)], 16, d.DTYPE_F32, y_dtype) >= _decode_ws_bytes(enc, k)
 
 
+@pytest.mark.parametrize("enc,rows,n,k", [
+    (d.ENC_Q4_0, 3, 16400, 16384), (d.ENC_Q4_K, 4, 16400, 16384), (d.ENC_Q6_K, 4, 16400, 16384),
+    (d.ENC_Q4_K, 8, 768, 12288), (d.ENC_Q5_K, 5, 600, 12288), (d.ENC_Q6_K, 7, 250, 7680)])
+def test_long_k_decode_stays_on_the_16_row_path(enc, rows, n, k):
+    """Where the activation tile of the 4x4 kernels does not fit LDS they take several passes
+    over the weights; the 16-row MFMA GEMV (K in several segments: staged in the workspace)
+    keeps the launches it serves faster."""
+    assert d.prefill_workspace_bytes([w(enc, n, k)], rows) == _decode_ws_bytes(enc, k)
+
+
 def test_prefill_workspace_bytes_validates_like_the_call():
     lib = d.library()
     arr = (d._QWeightC * 2)(w(d.ENC_Q4_0, 64, 1024).c(), w(d.ENC_Q4_0, 64, 512).c())

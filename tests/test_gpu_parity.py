@@ -235,6 +235,9 @@ def test_gemv_mfma(ctx, gtype, n, k, batch, ybf16, off):
 # from 8 MB or 1024 tiles: 1025 tiles, the oracle on the first 2048 rows.
 PRESTAGE_CASES = [c for c in MFMA_CASES if c[2] >= 2048 and (c[3] > 8 or c[2] > 4096)] + [
     (oracle.Q4_0, 16400, 8192, 5, False, 0), (oracle.Q4_K, 6144, 4096, 16, False, 0),
+    # 3..8 rows whose activation tile is too long for the 4x4 kernels' one pass
+    (oracle.Q4_0, 16400, 16384, 3, False, 0), (oracle.Q4_K, 768, 12288, 8, False, 0),
+    (oracle.Q6_K, 250, 7680, 7, False, 0), (oracle.Q5_K, 600, 12288, 5, False, 0),
     (oracle.Q5_K, 4096, 12288, 9, False, 0), (oracle.IQ4_XS, 6144, 2048, 12, True, 0),
     # split mode, 16 tasks per segment: each wave's staged operands in registers
     (oracle.Q4_0, 4096, 4096, 16, False, 0), (oracle.Q4_K, 4096, 12288, 16, False, 0),
