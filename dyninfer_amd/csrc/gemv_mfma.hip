@@ -1262,13 +1262,17 @@ bool gemv_mfma_applies(uint32_t enc, const GemvProblem* probs, int nprob, uint32
     // Q4_0 24576 x 16384 0.85 of its time), MLX and three rows of Q4_K from 1536 (16384 x
     // 16384 1.04 and 1.07 of theirs, 24576 0.96 and 0.95); 5..8 rows of 64-weight chunks from
     // seven rows or K = 8192 (768 x 12288 at 8 rows: Q4_K 13.6 us, 23.8, Q6_K 15.1, 21.4; K =
-    // 7680 at 5 rows, passes of four and one, 1.08 to 1.22 of their time).
+    // 7680 at 5 rows, passes of four and one, 1.08 to 1.22 of their time).  In one pass too
+    // 64-weight chunks stay here above 2048 rows of K > 2048, too many for four waves each
+    // there (Q4_K 3072 x 2560 at 8 rows 8.3 us, 9.6, Q5_K 2100 x 3584 9.8, 11.8, Q6_K 3072 x
+    // 3072 8.8, 10.5).
     const bool one_pass = xtile_bytes(enc, batch <= 4u ? 4u : 8u, K) <= kLdsBytes;
     if (batch <= 4u) {
         const uint32_t long_k = enc == ENC_MLX_U4 || (enc == ENC_Q4_K && batch == 3u) ? 1536u : kMfmaSplitTiles;
         if (one_pass ? enc != ENC_Q6_K || tiles < 4096u : tiles < long_k) return false;
     } else if (batch <= 8u && bytes < (8ull << 20) && tiles < kMfmaSplitTiles) {
-        if (!wide_chunks(enc) || one_pass || (batch < 7u && K < 8192u)) return false;
+        const bool many = rows > 2048u && K > 2048u;
+        if (!wide_chunks(enc) || (one_pass ? !many : batch < 7u && K < 8192u)) return false;
     }
     const uint32_t min_tiles = mfma_min_tiles(batch);
     const int mode = enc == ENC_Q4_0   ? mfma_mode<MfmaQ40>(K, tiles, y_bf16, min_tiles)

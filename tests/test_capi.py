@@ -199,11 +199,12 @@ def test_decode_workspace_is_zero_where_none_is_used(enc, rows, n, k, y_dtype):
 
 @pytest.mark.parametrize("enc,rows,n,k", [
     (d.ENC_Q4_0, 3, 16400, 16384), (d.ENC_Q4_K, 4, 16400, 16384), (d.ENC_Q6_K, 4, 16400, 16384),
-    (d.ENC_Q4_K, 8, 768, 12288), (d.ENC_Q5_K, 5, 600, 12288), (d.ENC_Q6_K, 7, 250, 7680)])
+    (d.ENC_Q4_K, 8, 768, 12288), (d.ENC_Q5_K, 5, 600, 12288), (d.ENC_Q6_K, 7, 250, 7680),
+    (d.ENC_Q4_K, 8, 2100, 5120), (d.ENC_Q6_K, 5, 2052, 4608)])
 def test_long_k_decode_stays_on_the_16_row_path(enc, rows, n, k):
     """Where the activation tile of the 4x4 kernels does not fit LDS they take several passes
     over the weights; the 16-row MFMA GEMV (K in several segments: staged in the workspace)
-    keeps the launches it serves faster."""
+    keeps the launches it serves faster, and more than 2048 rows of 64-weight chunks."""
     assert d.prefill_workspace_bytes([w(enc, n, k)], rows) == _decode_ws_bytes(enc, k)
 
 
