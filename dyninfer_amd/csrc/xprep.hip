@@ -38,17 +38,16 @@
 // of 8 elements (slot 8c + 2t + h: chunk c, step t, half h) that it holds in
 // registers between the max pass and the conversion; the waves' maxima meet in
 // LDS.  Bound: HBM / L2 traffic for many rows, one memory round trip for few, so
-// what counts is loads in flight: WPR grows until the launch has 16 waves per CU
-// or a lane one slot (below).  With one wave per row, which reread rows longer
+// what counts is loads in flight: WPR grows until a lane has one slot or the launch
+// enough waves (launch_xprep).  With one wave per row, which reread rows longer
 // than 12288, 45 f32 rows of 12288 took 18.2 us, now 5.3; 512 bf16 rows of 12288
 // 27.8 -> 11.7; 2048 f32 rows of 12288 113 -> 29.6 us (5.1 TB/s of reads and
 // writes); 45 rows of 4096 6.6 -> 4.8.
 // From kXprepWholeMinRows rows (there are enough of them), and from
-// kXprepPartsMinRows when K >= kXprepPartsMinK, eight rows share a workgroup and
+// kXprepPartsMinRows of longer rows, eight rows share a workgroup and
 // their slots leave as whole 128-byte lines; otherwise each lane stores its own
-// 16-byte slots, four rows or fewer to a workgroup (512 rows: K = 1024 3.6 us
-// against 3.9 by lines, K = 3072 6.0 against 6.4; K = 4096 6.9 against 6.2,
-// K = 12288 13.3 against 11.7).
+// 16-byte slots, four rows or fewer to a workgroup (512 rows of K = 12288 13.7 us
+// against 12.5 by lines).
 // NaN and inf: the row's scale is taken as 2^15 and the non-finite values
 // propagate to the row's outputs.
 #include "device_common.hpp"
@@ -218,7 +217,7 @@ __global__ __launch_bounds__((WPR > 4u ? WPR : 4u) * 64u) void xprep_kernel(cons
 // reads the others for the maximum only, so fewer rows than CUs·8 still fill
 // the chip (PARTS; otherwise one workgroup holds the rows whole).  The LDS tile holds SEG slots per lane, so a long part passes
 // through it in NR / SEG turns.
-constexpr uint32_t kXprepLinesRows = 8, kXprepWholeMinRows = 1024, kXprepPartsMinRows = 256, kXprepPartsMinK = 4096;
+constexpr uint32_t kXprepLinesRows = 8, kXprepWholeMinRows = 1024, kXprepPartsMinRows = 256;
 template <bool XBF16, uint32_t LAYOUT, int NR, int SEG, uint32_t WPR, bool PARTS>
 __global__ __launch_bounds__(kXprepLinesRows * WPR * 64) void xprep_lines_kernel(const void* __restrict__ x, uint32_t M,
                                                                                 uint32_t K, uint16_t* __restrict__ xh,
@@ -293,10 +292,14 @@ hipError_t launch_rows(const void* x, uint32_t M, uint32_t Mp, uint32_t K, uint1
 template <bool XBF16, uint32_t LAYOUT, uint32_t WPR>
 hipError_t launch_rows(const void* x, uint32_t M, uint32_t Mp, uint32_t K, uint16_t* xh, float* rs, hipStream_t st) {
     const uint32_t nr = (K / 8u + 64u * WPR - 1u) / (64u * WPR);  // slots per lane
+    constexpr int most = WPR < 4u ? 1 : WPR == 4u ? 4 : WPR == 8u ? 2 : 8;  // (launch_xprep's rule meets no more)
     if (nr <= 1u) return launch_rows<XBF16, LAYOUT, 1, WPR>(x, M, Mp, K, xh, rs, st);
-    if (nr <= 2u) return launch_rows<XBF16, LAYOUT, 2, WPR>(x, M, Mp, K, xh, rs, st);
-    if (nr <= 4u) return launch_rows<XBF16, LAYOUT, 4, WPR>(x, M, Mp, K, xh, rs, st);
-    if (nr <= 8u) return launch_rows<XBF16, LAYOUT, 8, WPR>(x, M, Mp, K, xh, rs, st);
+    if constexpr (most >= 2)
+        if (nr <= 2u) return launch_rows<XBF16, LAYOUT, 2, WPR>(x, M, Mp, K, xh, rs, st);
+    if constexpr (most >= 4)
+        if (nr <= 4u) return launch_rows<XBF16, LAYOUT, 4, WPR>(x, M, Mp, K, xh, rs, st);
+    if constexpr (most >= 8)
+        if (nr <= 8u) return launch_rows<XBF16, LAYOUT, 8, WPR>(x, M, Mp, K, xh, rs, st);
     return hipErrorInvalidValue;
 }
 template <bool XBF16, uint32_t LAYOUT, int NR, int SEG, uint32_t WPR, bool PARTS>
@@ -317,11 +320,20 @@ hipError_t launch_xprep(const void* x, uint32_t M, uint32_t K, uint16_t* xh, flo
         if (slots <= 64u) return launch_lines<XBF16, LAYOUT, 1, 1, 1, false>(x, M, Mp, K, xh, rs, st);
         if (slots <= 128u) return launch_lines<XBF16, LAYOUT, 1, 1, 2, false>(x, M, Mp, K, xh, rs, st);
         if (slots <= 256u) return launch_lines<XBF16, LAYOUT, 2, 2, 2, false>(x, M, Mp, K, xh, rs, st);
+        // many f32 rows fill the chip with one wave to a row, and more of them share a CU (3000
+        // rows of 3072: two waves 15.2 us, one 10.2; 4096 of 4096 19.8, 16.2; 2048 rows 11.7
+        // by one, 10.9; 3000 bf16 rows alike)
+        if (!XBF16 && Mp > 2048u && slots > 256u && slots <= 512u)
+            return launch_lines<XBF16, LAYOUT, 8, 8, 1, false>(x, M, Mp, K, xh, rs, st);
         if (slots <= 512u) return launch_lines<XBF16, LAYOUT, 4, 4, 2, false>(x, M, Mp, K, xh, rs, st);
         if (slots <= 1024u) return launch_lines<XBF16, LAYOUT, 8, 4, 2, false>(x, M, Mp, K, xh, rs, st);
         return launch_lines<XBF16, LAYOUT, 12, 4, 2, false>(x, M, Mp, K, xh, rs, st);
     }
-    if (Mp >= kXprepPartsMinRows && K >= kXprepPartsMinK) {
+    // (f32 rows up to 5120 from 641 of them: fewer are faster below, the whole call of 512
+    // rows of Q4_0 1024 x 4096 21.0 us in parts, 18.3 below, 1024 x 5120 25.3 and 21.3, Q8_0
+    // 400 x 1024 x 4096 22.6 and 19.5; 768 rows stage in 7.2 us in parts, 7.6 below, and
+    // 512 bf16 rows of 4096 in 5.3 and 5.8)
+    if (Mp >= kXprepPartsMinRows && K >= 4096u && (XBF16 || Mp > 640u || K > 5120u)) {
         // slots per workgroup so that the launch has about 256 of them
         const uint64_t want = ((uint64_t)slots * (Mp / kXprepLinesRows) + 255u) / 256u;
         if (want <= 64u) return launch_lines<XBF16, LAYOUT, 1, 1, 1, true>(x, M, Mp, K, xh, rs, st);
@@ -329,10 +341,12 @@ hipError_t launch_xprep(const void* x, uint32_t M, uint32_t K, uint16_t* xh, flo
         if (want <= 256u) return launch_lines<XBF16, LAYOUT, 2, 2, 2, true>(x, M, Mp, K, xh, rs, st);
         return launch_lines<XBF16, LAYOUT, 4, 4, 2, true>(x, M, Mp, K, xh, rs, st);
     }
-    // waves per row: 4096 waves in all (16 per CU), at least one slot per lane, at most eight
+    // waves per row: 4096 waves in all (16 per CU), at least one slot per lane, at most
+    // eight; 2500 for the f32 rows above, whose lanes then load two slots or four
     const uint32_t full = (K + 511u) / 512u;  // waves with one slot per lane
+    const uint32_t waves = K < 4096u ? 4096u : 2500u;
     uint32_t wpr = 1u;
-    while (wpr < 16u && ((wpr < full && wpr * Mp < 4096u) || 8u * wpr < full)) wpr *= 2u;
+    while (wpr < 16u && ((wpr < full && wpr * Mp < waves) || 8u * wpr < full)) wpr *= 2u;
     switch (wpr) {
         case 1: return launch_rows<XBF16, LAYOUT, 1>(x, M, Mp, K, xh, rs, st);
         case 2: return launch_rows<XBF16, LAYOUT, 2>(x, M, Mp, K, xh, rs, st);

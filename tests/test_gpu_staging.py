@@ -31,8 +31,10 @@ def weight(layout, n, k):
 
 @pytest.mark.parametrize("layout", ["nib", "byte", "word"])
 @pytest.mark.parametrize("rows,k", [
-    (33, 64), (40, 576), (45, 4096), (45, 12352), (61, 20480),      # one slot a lane: 1..16 waves a row
-    (250, 1088), (700, 2112), (255, 4160), (1000, 1024),            # several slots a lane
+    (33, 64), (40, 576), (45, 4096), (45, 8192), (45, 12352), (61, 20480),      # one slot a lane: 1..16 waves a row
+    (250, 1088), (700, 2112), (255, 4160), (1000, 1024),
+    (640, 4096), (630, 5120), (300, 4160), (390, 5120), (20, 33024),  # several slots a lane (f32)
+    (2052, 2112), (2100, 4096),                                     # eight rows, whole, a wave each (f32)
     (256, 4096), (257, 4160), (700, 8256), (500, 12288), (300, 20480),  # eight rows a workgroup, in parts
     (1024, 64), (1025, 512), (1030, 1088), (1024, 4160), (1050, 8256), (1024, 12288),  # eight rows, whole
     (1024, 12352),                                                  # too long to hold whole: parts again
