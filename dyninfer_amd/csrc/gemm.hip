@@ -64,8 +64,15 @@ bool gemm_supported(uint32_t enc, uint32_t N, uint32_t K, uint32_t M) {
 // with rounds = ceil(workgroups / 256), nc the 64-k chunks per wave, V the decode and
 // scale VALU of a chunk, w waves per SIMD, S' = S (the epilogue's LDS round trip of
 // the partial tiles), r = 0.75 where several workgroups fit a CU (small tiles of four
-// waves), otherwise 1.  The configuration it picks takes 0.9% longer on average than the best
-// of them (8% at the 95th percentile, 18% at worst).
+// waves), otherwise 1.  128x256 tiles of four waves (4, 2, 1, 4, 1), which take the
+// fewest bytes from L2 per MFMA beside the 256x256 ones, cost f = 0.84 + 0.0173 for each
+// copy of their four weight windows above 12 of that: timed over 1704 shapes (eight
+// encodings, M 17..4096) a planner without them took 8% longer on 72 and on none
+// less (Q4_0 1536 x 4096 x 4096 84 -> 68 us, 2048 x 4096 x 4096 90 -> 79, 1024 x 24576 x
+// 4096 230 -> 207, Q4_K 3000 x 2560 x 2560 69 -> 59); with Q6_K's eight copies a wave, of
+// scattered dwords, the 256x128 tiles that share windows stay (2048 x 3072 x 1024 33 us
+// against 41).  The configuration it picks takes 1.1% longer on average than the best of
+// them (8% at the 95th percentile, 31% at worst).
 GemmPlan gemm_plan(uint32_t enc, const uint32_t* N, int count, uint32_t K, uint32_t M) {
     const uint32_t mb = (M + 31u) / 32u, nchk = K / 64u;
     const double valu = 4.0 * gemm::decode_valu(enc) + gemm::scale_valu(enc);
@@ -82,7 +89,8 @@ GemmPlan gemm_plan(uint32_t enc, const uint32_t* N, int count, uint32_t K, uint3
         const double w = s * wn * wm / 4.0, tiles = tm * nb;
         const double wg = 1.04 + 0.101 * tiles * s +
                           nc * (0.00165 * nb * valu + 0.0673 * tiles + 0.38) * (1.0 + 0.37 * (w - 1.0));
-        const double t = 0.86 + wg * (1.0 + (tiles <= 4.0 && tm <= 2u && w == 1.0 ? 0.75 : 1.0) * (rounds - 1.0));
+        const double f = tm == 4u && wn == 4u ? 0.84 + 0.0173 * (4.0 * gemm::window_copies(enc) - 12.0) : 1.0;
+        const double t = f * (0.86 + wg * (1.0 + (tiles <= 4.0 && tm <= 2u && w == 1.0 ? 0.75 : 1.0) * (rounds - 1.0)));
         if (t < best_t * 0.999) {
             best_t = t;
             best = {tm, nb, s, wn, wm, mt, nt};

@@ -817,6 +817,11 @@ constexpr int scale_valu(uint32_t enc) {
     return enc == ENC_Q6_K || enc == ENC_Q4_K || enc == ENC_Q5_K ? 32 : enc == ENC_MLX_U4 ? 20 : enc == ENC_IQ4_XS ? 12 : 4;
 }
 
+// Copy instructions of a wave's window of two weight blocks (see WinOf).
+constexpr uint32_t window_copies(uint32_t enc) {
+    return enc == ENC_Q6_K ? 8u : enc == ENC_Q8_0 || enc == ENC_Q5_K ? 5u : enc == ENC_MLX_U4 ? 4u : 3u;
+}
+
 // LDS geometry of one kernel configuration: a wave multiplies TM activation
 // row blocks by NB weight row blocks (32 rows each); the workgroup's S·WN·WM waves
 // split into S K slices x WN column subtiles x WM row subtiles.
@@ -854,6 +859,7 @@ struct Geo {
     static constexpr uint32_t kRing = ring_bytes(R) > kEpi ? ring_bytes(R) : kEpi;
     static constexpr uint32_t kLds = kRing + kRs;
     static_assert((4u * TM) % WN == 0, "activation fragments split evenly over the slice's waves");
+    static_assert(WinOf<ENC, 2, 1>::type::kCopies == window_copies(ENC), "the launch plan's window copies");
 };
 
 // Issue order of a k step of MF MFMAs: one MFMA, then a share of the copies, the
@@ -1159,7 +1165,7 @@ hipError_t launch(const GemmArgs& a, hipStream_t st) {
 
 // The configurations built: X(TM, NB, S, WN, WM).
 #define DMX_GEMM_CONFIGS(X) \
-    X(8, 2, 1, 4, 1) X(4, 2, 1, 2, 2) X(2, 2, 1, 4, 1) \
+    X(8, 2, 1, 4, 1) X(4, 2, 1, 4, 1) X(4, 2, 1, 2, 2) X(2, 2, 1, 4, 1) \
     X(8, 2, 4, 1, 1) X(4, 3, 4, 1, 1) X(4, 2, 4, 1, 1) X(2, 3, 4, 1, 1) X(2, 2, 4, 1, 1) X(2, 1, 4, 1, 1) \
     X(1, 1, 4, 1, 1) X(1, 1, 8, 1, 1)
 

@@ -64,13 +64,17 @@ SHAPES = [
     (75, [8000, 900, 103], 256),  # 2 3 4 1 1
     (70, [14001], 512),         # 4 2 4 1 1
     (97, [19000, 1001], 768),   # 4 3 4 1 1
-    (131, [13000, 1003], 768),  # 8 2 4 1 1
+    (131, [13000, 1003], 768),  # 8 2 4 1 1, blocks of 32: 2 2 1 4 1
+    (150, [12601], 1024),       # 8 2 4 1 1
     (131, [9001], 256),         # 2 2 1 4 1
-    (257, [14002], 256),        # 4 2 1 2 2
+    (257, [14002], 256),        # 4 2 1 4 1, Q6_K 4 2 1 2 2
+    (68, [35081], 256),         # 4 2 1 4 1
+    (645, [10781], 256),        # 4 2 1 2 2
     (400, [20001], 256),        # 8 2 1 4 1
     (400, [20001], 1024),       # the two above over a ring's worth of chunks
     (513, [6000, 3001], 1280),
 ]
+ODD_SHAPES = [(40, [97], 64), (41, [260, 30], 192), (70, [513], 320), (90, [1000], 1088), (300, [20000], 64)]
 
 
 @pytest.mark.parametrize("kind", BLOCKS + SUPER)
@@ -80,8 +84,7 @@ def test_gemm_plans(ctx, kind, m, ns, k):
 
 
 @pytest.mark.parametrize("kind", BLOCKS)
-@pytest.mark.parametrize("m,ns,k", [(40, [97], 64), (41, [260, 30], 192), (70, [513], 320), (90, [1000], 1088),
-                                    (300, [20000], 64)])
+@pytest.mark.parametrize("m,ns,k", ODD_SHAPES)
 def test_gemm_plans_odd_chunks(ctx, kind, m, ns, k):
     check(ctx, kind, m, ns, k)
 
@@ -117,7 +120,8 @@ def _shifted(a, off):
     (160, 45, [131], 960),    # 1 1 8 1 1
     (96, 45, [131], 960),
     (160, 20, [1000], 320),   # fewer rows than a row block
-    (96, 257, [14002], 192),  # 4 2 1 2 2: one of the two waves of a window copies the scales, one the biases
+    (96, 257, [14002], 192),  # 4 2 1 4 1
+    (96, 682, [10865], 192),  # 4 2 1 2 2: one of the two waves of a window copies the scales, one the biases
     (160, 260, [14002], 320),
 ])
 def test_gemm_mlx_groups_across_chunks(ctx, sdtype, off, group, m, ns, k):
