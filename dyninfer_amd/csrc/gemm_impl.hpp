@@ -850,7 +850,8 @@ struct Geo {
     // Vector memory operations newer than chunk c + 1's copies at step c's wait (at
     // least; XR: the activation loads of half a step besides the copies).
     static constexpr uint32_t kNewer = XR ? (R - 3u) * (4u * TM + kDma) + 2u * TM : (R - 3u) * kDma;
-    static constexpr bool kFits = ring_bytes(R) <= kRoom && kEpiBlock <= kRoom && (R - 2u) * kDma < 64u && kNewer < 64u;
+    static constexpr bool kFits = (S != 2 || window_copies(ENC) == 3u) &&  // (gemm_plan's only use of two slices)
+                                  ring_bytes(R) <= kRoom && kEpiBlock <= kRoom && (R - 2u) * kDma < 64u && kNewer < 64u;
     // the epilogue reuses the ring: row blocks of the tile per pass
     static constexpr uint32_t kEpiPer = S == 1 ? 1u
                                       : TM % 4 == 0 && 4u * kEpiBlock <= ring_bytes(R) ? 4u
@@ -1165,7 +1166,7 @@ hipError_t launch(const GemmArgs& a, hipStream_t st) {
 
 // The configurations built: X(TM, NB, S, WN, WM).
 #define DMX_GEMM_CONFIGS(X) \
-    X(8, 2, 1, 4, 1) X(4, 2, 1, 4, 1) X(4, 2, 1, 2, 2) X(2, 2, 1, 4, 1) \
+    X(8, 2, 1, 4, 1) X(4, 2, 1, 4, 1) X(4, 2, 1, 2, 2) X(2, 2, 1, 4, 1) X(4, 2, 2, 2, 1) \
     X(8, 2, 4, 1, 1) X(4, 3, 4, 1, 1) X(4, 2, 4, 1, 1) X(2, 3, 4, 1, 1) X(2, 2, 4, 1, 1) X(2, 1, 4, 1, 1) \
     X(1, 1, 4, 1, 1) X(1, 1, 8, 1, 1)
 

@@ -70,6 +70,7 @@ SHAPES = [
     (257, [14002], 256),        # 4 2 1 4 1, Q6_K 4 2 1 2 2
     (68, [35081], 256),         # 4 2 1 4 1
     (645, [10781], 256),        # 4 2 1 2 2
+    (3206, [867], 1024),        # 4 2 2 2 1, more copies a window: 8 2 4 1 1
     (400, [20001], 256),        # 8 2 1 4 1
     (400, [20001], 1024),       # the two above over a ring's worth of chunks
     (513, [6000, 3001], 1280),
