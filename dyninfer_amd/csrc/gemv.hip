@@ -196,8 +196,9 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
         // would leave most SIMDs idle: four waves share one (us per launch, one wave
         // against four: MLX 1024 x 3072 at 8 rows 8.8 -> 6.5, Q8_0 10.8 -> 8.6, Q6_K
         // 1024 x 4096 at 4 rows 7.6 -> 5.1, 2048 x 14336 18.8 -> 14.5, Q4_0 4096 x 4096
-        // 6.5 -> 6.2; but 4096 x 1024 4.1 -> 4.8 and 4096 x 4096 at 8 rows 9.7 -> 11.9:
-        // every workgroup stages the activations).  Where these leave one workgroup per
+        // 6.5 -> 6.2; the pipeline against four, IQ4_XS 2048 x 6144 at 8 rows 13.2 -> 9.0,
+        // Q8_0 18.1 -> 13.0; but 4096 x 1024 4.1 -> 4.8 and 4096 x 4096 at 8 rows 9.7 ->
+        // 11.9: every workgroup stages the activations).  Where these leave one workgroup per
         // CU it has four row blocks, all its loads in flight at once (4 rows, the
         // pipeline against this: Q4_0 4096 x 12288 17.3 -> 14.0, Q4_K 17.2 -> 15.8, Q6_K
         // 20.3 -> 19.2, Q8_0 -> 20.2, Q4_K 4096 x 8192 13.3 -> 10.9), while the CUs take
@@ -210,10 +211,10 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
         const uint32_t cps = (nch + 63u) / 64u;  // chunks per lane, four waves per row block
         const uint32_t cpw = info.wide ? (nch + 31u) / 32u : cps;
         const bool one_per_cu = tile > kLdsBytes / 2u;
-        const uint32_t max_cps = B == 4u ? (info.wide ? 4u : 8u) : 2u;
+        const uint32_t max_cps = B == 4u ? (info.wide ? 4u : 8u) : info.wide ? 2u : 4u;
         if (tile + kSplitSums <= lim &&
             ((rbs1 <= 512u && cps <= max_cps) || (B == 4u && rbs1 <= 1024u && K >= 2048u && cps <= 2u && !one_per_cu)))
-            oneshot = kOneshotSplit | (cps <= 2u ? cps : cps <= 4u ? 4u : 8u);
+            oneshot = kOneshotSplit | cps;
         else if (B == 4u && rbs1 <= 1024u && one_per_cu && tile + kSplitSums <= lim && cpw <= (info.wide ? 6u : 7u))
             oneshot = kOneshotWide | (cpw <= 4u ? 4u : cpw <= 6u ? 6u : 7u);
         else if (cpl <= 2u) oneshot = rbs1 <= 8192u ? cpl : 0u;

@@ -1304,7 +1304,10 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
         DMX_ONESHOT(8, 1)
         DMX_ONESHOT(8, 2)
         DMX_ONESHOT(8, 4)
-        // four waves per row block: kOneshotSplit besides the chunks per lane
+        // four waves per row block: kOneshotSplit besides the chunks per lane, exactly (a
+        // lane with one chunk more than the row has loads and multiplies it for nothing:
+        // Q5_K 2048 x 12288 at 4 bf16 rows 14.3 us with 4 chunks a lane, 12.7 with 3, Q8_0
+        // 2048 x 10240 13.1 with 8, 11.5 with 5)
 #define DMX_ONESHOT_SPLIT(b, c)                                                                       \
     if (B == b && oneshot == (kOneshotSplit | c))                                                     \
         return launch_oneshot(gguf_gemv_oneshot_kernel<E, c, b, xmode_rows(XM, b), 512, 4>,           \
@@ -1314,6 +1317,7 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
         return launch_oneshot_wide(gguf_gemv_oneshot_kernel<E, c, 4, xmode_rows(XM, 4), th, th / 256>, p, lds, st, th);
         DMX_ONESHOT_SPLIT(4, 1)
         DMX_ONESHOT_SPLIT(4, 2)
+        DMX_ONESHOT_SPLIT(4, 3)
         DMX_ONESHOT_SPLIT(4, 4)
         DMX_ONESHOT_SPLIT(8, 1)
         DMX_ONESHOT_SPLIT(8, 2)
@@ -1321,7 +1325,12 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
             DMX_ONESHOT_WIDE(4, 512)
             DMX_ONESHOT_WIDE(6, 512)
         } else {
-            DMX_ONESHOT_SPLIT(4, 8)
+            DMX_ONESHOT_SPLIT(4, 5)
+            DMX_ONESHOT_SPLIT(4, 6)
+            DMX_ONESHOT_SPLIT(4, 7)
+            if constexpr (xtile_chunk_bytes(E::ENC) < 96u) DMX_ONESHOT_SPLIT(4, 8)
+            DMX_ONESHOT_SPLIT(8, 3)
+            DMX_ONESHOT_SPLIT(8, 4)
             DMX_ONESHOT_WIDE(4, 1024)
             DMX_ONESHOT_WIDE(6, 1024)
             DMX_ONESHOT_WIDE(7, 1024)

@@ -36,10 +36,15 @@ hipError_t launch_mlx(const GemvParams& p, uint32_t B, uint32_t oneshot, hipStre
         return launch_oneshot_wide(mlx_u4_gemv_oneshot_kernel<c, 4, xmode_rows(XM, 4), 1024, 4>, p, lds, st, 1024);
         DMX_ONESHOT_SPLIT(4, 1)
         DMX_ONESHOT_SPLIT(4, 2)
+        DMX_ONESHOT_SPLIT(4, 3)
         DMX_ONESHOT_SPLIT(4, 4)
-        DMX_ONESHOT_SPLIT(4, 8)
+        DMX_ONESHOT_SPLIT(4, 5)
+        DMX_ONESHOT_SPLIT(4, 6)
+        DMX_ONESHOT_SPLIT(4, 7)
         DMX_ONESHOT_SPLIT(8, 1)
         DMX_ONESHOT_SPLIT(8, 2)
+        DMX_ONESHOT_SPLIT(8, 3)
+        DMX_ONESHOT_SPLIT(8, 4)
         DMX_ONESHOT_WIDE(4)
         DMX_ONESHOT_WIDE(6)
         DMX_ONESHOT_WIDE(7)

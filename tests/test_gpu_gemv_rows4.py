@@ -61,8 +61,28 @@ SHAPES = [
     (4, [1030, 250], 7936),       # ... four
     (4, [1500], 14336),           # four waves per row block, up to eight chunks a lane
     (3, [1026], 6144),
+    (4, [1501], 10240),           # ... three and five
+    (3, [1030], 14592),           # ... and eight, where the tile fits
+    (4, [2043], 14080),           # ... seven
+    (3, [1027, 900], 512),        # a wave each, one chunk a lane
+    (5, [997], 4352),             # eight rows, four waves per row block, three chunks a lane
+    (7, [2047], 6656),            # ... four
+    (4, [2100], 8192),            # three row blocks to a workgroup, four chunks a lane
+    (3, [2501], 10240),           # ... five
+    (4, [3070], 12288),           # ... six
+    (4, [2053], 13312),           # ... seven
+    (3, [3075], 10240),           # four, five chunks a lane
+    (4, [4095], 8192),            # ... four
+    (8, [2101], 5120),            # eight rows: three, three chunks a lane
+    (6, [2103], 6656),            # ... four
+    (8, [3333], 6144),            # four row blocks, three chunks a lane (of Q8_0 and Q4_1)
+    (8, [4001], 6656),
+    (4, [3071], 2560),            # 64-weight chunks: the pipeline
+    (3, [2301], 7168),
+    (4, [3333], 9216),
+    (8, [2500], 2560),            # 64-weight chunks: the 16-row kernels
     (4, [8200], 7680),            # one workgroup to a CU, more row blocks than they take at once
-    (8, [2100], 5120),            # the pipeline, one workgroup to a CU
+    (8, [2100, 2200], 5120),      # the pipeline, one workgroup to a CU
     (4, [33001], 256),
     (8, [8197, 8197], 768),
     (16, [517], 1280),            # two passes, or the 16-row kernels
