@@ -198,7 +198,8 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
         // 1024 x 4096 at 4 rows 7.6 -> 5.1, 2048 x 14336 18.8 -> 14.5, Q4_0 4096 x 4096
         // 6.5 -> 6.2; the pipeline against four, IQ4_XS 2048 x 6144 at 8 rows 13.2 -> 9.0,
         // Q8_0 18.1 -> 13.0; but 4096 x 1024 4.1 -> 4.8 and 4096 x 4096 at 8 rows 9.7 ->
-        // 11.9: every workgroup stages the activations).  Where these leave one workgroup per
+        // 11.9: every workgroup stages the activations; and of one chunk a lane, from
+        // 256 row blocks, Q5_K 2048 x 512 3.2 -> 4.2).  Where these leave one workgroup per
         // CU it has four row blocks, all its loads in flight at once (4 rows, the
         // pipeline against this: Q4_0 4096 x 12288 17.3 -> 14.0, Q4_K 17.2 -> 15.8, Q6_K
         // 20.3 -> 19.2, Q8_0 -> 20.2, Q4_K 4096 x 8192 13.3 -> 10.9), while the CUs take
@@ -213,7 +214,7 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
         const bool one_per_cu = tile > kLdsBytes / 2u;
         const uint32_t max_cps = B == 4u ? (info.wide ? 4u : 8u) : info.wide ? 2u : 4u;
         if (tile + kSplitSums <= lim &&
-            ((rbs1 <= 512u && cps <= max_cps) || (B == 4u && rbs1 <= 1024u && K >= 2048u && cps <= 2u && !one_per_cu)))
+            ((rbs1 <= 512u && cps <= max_cps && !(B == 4u && rbs1 > 256u && cpl == 1u)) || (B == 4u && rbs1 <= 1024u && K >= 2048u && cps <= 2u && !one_per_cu)))
             oneshot = kOneshotSplit | cps;
         else if (B == 4u && rbs1 <= 1024u && one_per_cu && tile + kSplitSums <= lim && cpw <= (info.wide ? 6u : 7u))
             oneshot = kOneshotWide | (cpw <= 4u ? 4u : cpw <= 6u ? 6u : 7u);
