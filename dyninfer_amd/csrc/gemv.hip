@@ -192,32 +192,38 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
     uint32_t oneshot = cpl >= 1 && cpl <= max_cpl && rbs1 <= max_rbs ? cpl : 0u;
     if (B >= 4) {
         // 4 and 8 rows, a row block being four rows by sixteen lanes.  Up to 512 row
-        // blocks (1024 at 4 rows from K = 2048, two workgroups to a CU) one wave each
-        // would leave most SIMDs idle: four waves share one (us per launch, one wave
-        // against four: MLX 1024 x 3072 at 8 rows 8.8 -> 6.5, Q8_0 10.8 -> 8.6, Q6_K
-        // 1024 x 4096 at 4 rows 7.6 -> 5.1, 2048 x 14336 18.8 -> 14.5, Q4_0 4096 x 4096
-        // 6.5 -> 6.2; the pipeline against four, IQ4_XS 2048 x 6144 at 8 rows 13.2 -> 9.0,
-        // Q8_0 18.1 -> 13.0; but 4096 x 1024 4.1 -> 4.8 and 4096 x 4096 at 8 rows 9.7 ->
-        // 11.9: every workgroup stages the activations; and of one chunk a lane, from
-        // 256 row blocks, Q5_K 2048 x 512 3.2 -> 4.2).  Where these leave one workgroup per
-        // CU it has four row blocks, all its loads in flight at once (4 rows, the
-        // pipeline against this: Q4_0 4096 x 12288 17.3 -> 14.0, Q4_K 17.2 -> 15.8, Q6_K
-        // 20.3 -> 19.2, Q8_0 -> 20.2, Q4_K 4096 x 8192 13.3 -> 10.9), while the CUs take
-        // all row blocks at once (Q4_K 8192 x 12288, two rounds, 20.0 -> 29.2) and the
-        // chunks fit the registers (Q5_K 4096 x 14336, eight a lane, 24.0 -> 27.0).  One
-        // wave per row block up to 8192 of them at 1..2 chunks per lane (MLX 6144 x 1024
+        // blocks (1024 at 4 rows from K = 2048, two workgroups to a CU) one wave each would leave most SIMDs idle: four waves share one (us per
+        // launch, one wave against four: MLX 1024 x 3072 at 8 rows 8.8 -> 6.5, Q8_0 10.8 ->
+        // 8.6, Q6_K 1024 x 4096 at 4 rows 7.6 -> 5.1, 2048 x 14336 18.8 -> 14.5, Q4_0 4096 x
+        // 4096 6.5 -> 6.2; the pipeline against four, IQ4_XS 2048 x 6144 at 8 rows 13.2
+        // -> 9.0, Q8_0 18.1 -> 13.0; but 4096 x 1024 4.1 -> 4.8: every workgroup stages the
+        // activations; and of one chunk a lane, from 256 row blocks, Q5_K 2048 x 512 3.2 ->
+        // 4.2).
+        const uint64_t tile = xtile_bytes(enc, B, K);
+        const bool room = tile + kSplitSums <= lim, one_per_cu = tile > kLdsBytes / 2u;
+        const uint32_t cps = (nch + 63u) / 64u;  // chunks per lane, four waves per row block
+        const uint32_t cpw = (nch + 31u) / 32u;  // ... two
+        const uint32_t max_cps = B == 4u ? (info.wide ? 4u : 8u) : info.wide ? 2u : 4u;
+        if (room && ((rbs1 <= 512u && cps <= max_cps && !(B == 4u && rbs1 > 256u && cpl == 1u)) ||
+                     (B == 4u && rbs1 <= 1024u && K >= 2048u && cps <= 2u && !one_per_cu)))
+            oneshot = kOneshotSplit | cps;
+        // More row blocks where the tile leaves one workgroup per CU: three to a workgroup,
+        // four from 768, all their loads in flight at once, while the CUs take all of them
+        // in one round (us per launch at 4 rows, the pipeline, four and three to a
+        // workgroup: Q4_0 2100 x 9216 11.9, 9.8, 8.5, Q8_0 3072 x 10240 21.2, 15.8, 14.6,
+        // IQ4_XS 2500 x 12288 18.2, 16.5, 13.6, Q4_0 4096 x 12288 in four 17.4 -> 13.6; at 8
+        // rows Q8_0 3000 x 6144 18.6, 15.8, 14.6, but bf16 13.7, 16.2, 14.1).
+        else if (!info.wide && room && one_per_cu && rbs1 <= 1024u && cps >= (B == 4u ? 4u : 3u) &&
+                 cps <= (B == 4u ? 7u : 4u) && !(B == 8u && enc == ENC_Q8_0 && x_bf16))
+            oneshot = (rbs1 <= 768u ? kOneshotThree : kOneshotWide) | cps;
+        // 64-weight chunks: four row blocks of two waves each (4 rows, the pipeline against
+        // these: Q4_K 4096 x 12288 17.2 -> 15.8, Q6_K 20.3 -> 19.2, Q4_K 4096 x 8192 13.3 ->
+        // 10.9; but Q5_K 4096 x 14336, eight chunks a lane, 24.0 -> 27.0).
+        else if (B == 4u && info.wide && rbs1 <= 1024u && one_per_cu && room && cpw <= 6u)
+            oneshot = kOneshotWide | (cpw <= 4u ? 4u : 6u);
+        // One wave per row block up to 8192 of them at 1..2 chunks per lane (MLX 6144 x 1024
         // at 8 rows 5.8 us in the pipeline, 5.3) and 2048 at more (Q4_0 6144 x 4096 at 4
         // rows 10.2 against 8.0; Q4_0 24576 x 4096 16.4 against 20.5).
-        const uint64_t tile = xtile_bytes(enc, B, K);
-        const uint32_t cps = (nch + 63u) / 64u;  // chunks per lane, four waves per row block
-        const uint32_t cpw = info.wide ? (nch + 31u) / 32u : cps;
-        const bool one_per_cu = tile > kLdsBytes / 2u;
-        const uint32_t max_cps = B == 4u ? (info.wide ? 4u : 8u) : info.wide ? 2u : 4u;
-        if (tile + kSplitSums <= lim &&
-            ((rbs1 <= 512u && cps <= max_cps && !(B == 4u && rbs1 > 256u && cpl == 1u)) || (B == 4u && rbs1 <= 1024u && K >= 2048u && cps <= 2u && !one_per_cu)))
-            oneshot = kOneshotSplit | cps;
-        else if (B == 4u && rbs1 <= 1024u && one_per_cu && tile + kSplitSums <= lim && cpw <= (info.wide ? 6u : 7u))
-            oneshot = kOneshotWide | (cpw <= 4u ? 4u : cpw <= 6u ? 6u : 7u);
         else if (cpl <= 2u) oneshot = rbs1 <= 8192u ? cpl : 0u;
         else oneshot = rbs1 <= 2048u && cpl <= (info.wide ? 4u : 8u) ? (cpl <= 4u ? 4u : 8u) : 0u;
     }

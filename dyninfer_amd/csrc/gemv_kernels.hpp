@@ -1252,14 +1252,14 @@ hipError_t launch_oneshot(KERNEL k512, KERNEL k256, GemvParams p, size_t lds, hi
     return hipGetLastError();
 }
 
-// Latency mode with four row blocks to a workgroup: of 1024 threads, four waves per row
-// block, or of 512, two.
-inline hipError_t launch_oneshot_wide(GemvKernel k, GemvParams p, size_t lds, hipStream_t st, unsigned threads) {
+// Latency mode with nrb row blocks to a workgroup of `threads` threads.
+inline hipError_t launch_oneshot_wide(GemvKernel k, GemvParams p, size_t lds, hipStream_t st, unsigned threads,
+                                      unsigned nrb) {
     int cus = 0, per_cu = 0;
     const hipError_t e = cached_occupancy(reinterpret_cast<const void*>(k), lds, (int)threads, &per_cu, &cus);
     if (e != hipSuccess) return e;
     layout_row_blocks(p, 64u >> p.lanes_log2);
-    p.grid = (p.total_rb + 3u) / 4u;
+    p.grid = (p.total_rb + nrb - 1u) / nrb;
     hipLaunchKernelGGL(k, dim3(p.grid), dim3(threads), lds, st, p);
     return hipGetLastError();
 }
@@ -1312,9 +1312,12 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
     if (B == b && oneshot == (kOneshotSplit | c))                                                     \
         return launch_oneshot(gguf_gemv_oneshot_kernel<E, c, b, xmode_rows(XM, b), 512, 4>,           \
                               gguf_gemv_oneshot_kernel<E, c, b, xmode_rows(XM, b), 256, 4>, p, lds, st, 4u);
-#define DMX_ONESHOT_WIDE(c, th)                                                                       \
-    if (B == 4 && oneshot == (kOneshotWide | c))                                                      \
-        return launch_oneshot_wide(gguf_gemv_oneshot_kernel<E, c, 4, xmode_rows(XM, 4), th, th / 256>, p, lds, st, th);
+#define DMX_ONESHOT_WIDE(b, c, mode, nrb, th)                                                         \
+    if (B == b && oneshot == (mode | c))                                                              \
+        return launch_oneshot_wide(gguf_gemv_oneshot_kernel<E, c, b, xmode_rows(XM, b), th, th / 64 / nrb>, p, lds, \
+                                   st, th, nrb);
+#define DMX_ONESHOT_FOUR_THREE(b, c) \
+    DMX_ONESHOT_WIDE(b, c, kOneshotWide, 4, 1024) DMX_ONESHOT_WIDE(b, c, kOneshotThree, 3, 768)
         DMX_ONESHOT_SPLIT(4, 1)
         DMX_ONESHOT_SPLIT(4, 2)
         DMX_ONESHOT_SPLIT(4, 3)
@@ -1322,8 +1325,8 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
         DMX_ONESHOT_SPLIT(8, 1)
         DMX_ONESHOT_SPLIT(8, 2)
         if constexpr (wide_chunks(E::ENC)) {
-            DMX_ONESHOT_WIDE(4, 512)
-            DMX_ONESHOT_WIDE(6, 512)
+            DMX_ONESHOT_WIDE(4, 4, kOneshotWide, 4, 512)
+            DMX_ONESHOT_WIDE(4, 6, kOneshotWide, 4, 512)
         } else {
             DMX_ONESHOT_SPLIT(4, 5)
             DMX_ONESHOT_SPLIT(4, 6)
@@ -1331,10 +1334,14 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
             if constexpr (xtile_chunk_bytes(E::ENC) < 96u) DMX_ONESHOT_SPLIT(4, 8)
             DMX_ONESHOT_SPLIT(8, 3)
             DMX_ONESHOT_SPLIT(8, 4)
-            DMX_ONESHOT_WIDE(4, 1024)
-            DMX_ONESHOT_WIDE(6, 1024)
-            DMX_ONESHOT_WIDE(7, 1024)
+            DMX_ONESHOT_FOUR_THREE(4, 4)
+            DMX_ONESHOT_FOUR_THREE(4, 5)
+            DMX_ONESHOT_FOUR_THREE(4, 6)
+            DMX_ONESHOT_FOUR_THREE(4, 7)
+            DMX_ONESHOT_FOUR_THREE(8, 3)
+            DMX_ONESHOT_FOUR_THREE(8, 4)
         }
+#undef DMX_ONESHOT_FOUR_THREE
 #undef DMX_ONESHOT_WIDE
 #undef DMX_ONESHOT_SPLIT
         if constexpr (!wide_chunks(E::ENC)) {

@@ -31,9 +31,11 @@ hipError_t launch_mlx(const GemvParams& p, uint32_t B, uint32_t oneshot, hipStre
     if (B == b && oneshot == (kOneshotSplit | c))                                                          \
         return launch_oneshot(mlx_u4_gemv_oneshot_kernel<c, b, xmode_rows(XM, b), 512, 4>,                  \
                               mlx_u4_gemv_oneshot_kernel<c, b, xmode_rows(XM, b), 256, 4>, p, lds, st, 4u);
-#define DMX_ONESHOT_WIDE(c)                                                                                \
-    if (B == 4 && oneshot == (kOneshotWide | c))                                                           \
-        return launch_oneshot_wide(mlx_u4_gemv_oneshot_kernel<c, 4, xmode_rows(XM, 4), 1024, 4>, p, lds, st, 1024);
+#define DMX_ONESHOT_WIDE(b, c, mode, nrb, th)                                                              \
+    if (B == b && oneshot == (mode | c))                                                                   \
+        return launch_oneshot_wide(mlx_u4_gemv_oneshot_kernel<c, b, xmode_rows(XM, b), th, 4>, p, lds, st, th, nrb);
+#define DMX_ONESHOT_FOUR_THREE(b, c) \
+    DMX_ONESHOT_WIDE(b, c, kOneshotWide, 4, 1024) DMX_ONESHOT_WIDE(b, c, kOneshotThree, 3, 768)
         DMX_ONESHOT_SPLIT(4, 1)
         DMX_ONESHOT_SPLIT(4, 2)
         DMX_ONESHOT_SPLIT(4, 3)
@@ -45,9 +47,13 @@ hipError_t launch_mlx(const GemvParams& p, uint32_t B, uint32_t oneshot, hipStre
         DMX_ONESHOT_SPLIT(8, 2)
         DMX_ONESHOT_SPLIT(8, 3)
         DMX_ONESHOT_SPLIT(8, 4)
-        DMX_ONESHOT_WIDE(4)
-        DMX_ONESHOT_WIDE(6)
-        DMX_ONESHOT_WIDE(7)
+        DMX_ONESHOT_FOUR_THREE(4, 4)
+        DMX_ONESHOT_FOUR_THREE(4, 5)
+        DMX_ONESHOT_FOUR_THREE(4, 6)
+        DMX_ONESHOT_FOUR_THREE(4, 7)
+        DMX_ONESHOT_FOUR_THREE(8, 3)
+        DMX_ONESHOT_FOUR_THREE(8, 4)
+#undef DMX_ONESHOT_FOUR_THREE
 #undef DMX_ONESHOT_WIDE
 #undef DMX_ONESHOT_SPLIT
 #undef DMX_ONESHOT

@@ -77,8 +77,9 @@ __host__ __device__ constexpr uint64_t xtile_bytes(uint32_t enc, uint32_t B, uin
 // run as several launches).
 __host__ __device__ constexpr uint32_t max_register_batch(uint32_t) { return 8u; }
 // Latency mode with four waves per row block (with the chunks per lane in the low bits).
-// kOneshotWide: in workgroups of 1024 threads (64-weight chunks: two waves, of 512).
-constexpr uint32_t kOneshotSplit = 0x100u, kOneshotWide = 0x200u;
+// kOneshotWide: four row blocks to a workgroup (64-weight chunks: of two waves each);
+// kOneshotThree: three.
+constexpr uint32_t kOneshotSplit = 0x100u, kOneshotWide = 0x200u, kOneshotThree = 0x400u;
 constexpr uint32_t kSplitSums = 2048u;  // LDS of their sums besides the activation tile, at most
 // LDS of one gfx950 workgroup.
 constexpr uint32_t kLdsBytes = 160u * 1024u;
