@@ -192,7 +192,8 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
     uint32_t oneshot = cpl >= 1 && cpl <= max_cpl && rbs1 <= max_rbs ? cpl : 0u;
     if (B >= 4) {
         // 4 and 8 rows, a row block being four rows by sixteen lanes.  Up to 512 row
-        // blocks (1024 at 4 rows from K = 2048, two workgroups to a CU) one wave each would leave most SIMDs idle: four waves share one (us per
+        // blocks (of 32-weight chunks 1024 at 4 rows from K = 2048, two workgroups to a
+        // CU) one wave each would leave most SIMDs idle: four waves share one (us per
         // launch, one wave against four: MLX 1024 x 3072 at 8 rows 8.8 -> 6.5, Q8_0 10.8 ->
         // 8.6, Q6_K 1024 x 4096 at 4 rows 7.6 -> 5.1, 2048 x 14336 18.8 -> 14.5, Q4_0 4096 x
         // 4096 6.5 -> 6.2; the pipeline against four, IQ4_XS 2048 x 6144 at 8 rows 13.2
@@ -202,10 +203,9 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
         const uint64_t tile = xtile_bytes(enc, B, K);
         const bool room = tile + kSplitSums <= lim, one_per_cu = tile > kLdsBytes / 2u;
         const uint32_t cps = (nch + 63u) / 64u;  // chunks per lane, four waves per row block
-        const uint32_t cpw = (nch + 31u) / 32u;  // ... two
         const uint32_t max_cps = B == 4u ? (info.wide ? 4u : 8u) : info.wide ? 2u : 4u;
         if (room && ((rbs1 <= 512u && cps <= max_cps && !(B == 4u && rbs1 > 256u && cpl == 1u)) ||
-                     (B == 4u && rbs1 <= 1024u && K >= 2048u && cps <= 2u && !one_per_cu)))
+                     (B == 4u && !info.wide && rbs1 <= 1024u && K >= 2048u && cps <= 2u && !one_per_cu)))
             oneshot = kOneshotSplit | cps;
         // More row blocks where the tile leaves one workgroup per CU: three to a workgroup,
         // four from 768, all their loads in flight at once, while the CUs take all of them
@@ -216,11 +216,17 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
         else if (!info.wide && room && one_per_cu && rbs1 <= 1024u && cps >= (B == 4u ? 4u : 3u) &&
                  cps <= (B == 4u ? 7u : 4u) && !(B == 8u && enc == ENC_Q8_0 && x_bf16))
             oneshot = (rbs1 <= 768u ? kOneshotThree : kOneshotWide) | cps;
-        // 64-weight chunks: four row blocks of two waves each (4 rows, the pipeline against
-        // these: Q4_K 4096 x 12288 17.2 -> 15.8, Q6_K 20.3 -> 19.2, Q4_K 4096 x 8192 13.3 ->
-        // 10.9; but Q5_K 4096 x 14336, eight chunks a lane, 24.0 -> 27.0).
-        else if (B == 4u && info.wide && rbs1 <= 1024u && one_per_cu && room && cpw <= 6u)
-            oneshot = kOneshotWide | (cpw <= 4u ? 4u : 6u);
+        // 64-weight chunks at 4 rows, 513 to 1024 row blocks: the pipeline (four waves each
+        // against it, two workgroups to a CU: Q4_K 3072 x 2560 8.0 -> 6.2, 3072 x 7168 15.8 ->
+        // 10.7, Q6_K bf16 3072 x 7168 15.8 -> 11.2), and for f32 rows of one workgroup to a
+        // CU with four or six chunks a lane four row blocks of two waves (the pipeline
+        // against them: Q4_K 4096 x 8192 11.7 -> 10.6, 4096 x 12288 16.6 -> 15.1, Q6_K 4096 x
+        // 8192 12.5 -> 12.3; bf16 Q5_K 4096 x 12288 16.1 against 18.5, five chunks, Q6_K f32
+        // 4096 x 9216 14.4 against 14.9).
+        else if (B == 4u && info.wide && K >= 2048u && rbs1 <= 1024u) {
+            const uint32_t cpw = (nch + 31u) / 32u;
+            oneshot = room && one_per_cu && !x_bf16 && (cpw == 4u || cpw == 6u) ? kOneshotWide | cpw : 0u;
+        }
         // One wave per row block up to 8192 of them at 1..2 chunks per lane (MLX 6144 x 1024
         // at 8 rows 5.8 us in the pipeline, 5.3) and 2048 at more (Q4_0 6144 x 4096 at 4
         // rows 10.2 against 8.0; Q4_0 24576 x 4096 16.4 against 20.5).
