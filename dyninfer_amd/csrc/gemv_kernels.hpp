@@ -82,23 +82,33 @@ template <class E, int B>
 __device__ __forceinline__ uint32_t xrow_dwords(uint32_t nch) {
     return nch * XTile<E>::XPW + (kM4<B> ? kXRowSkew / 4u : 0u);
 }
+// Offset of a staged chunk in the tile: by its number where the rows are not skewed (one
+// multiplication a staging thread: two rows of Q4_0 151936 x 1024 took 24.4 us with two,
+// 22.9 with one, IQ4_XS 32.9 and 30.7), but for 64-weight chunks, whose two-row tiles come out
+// at other register counts (Q4_K 13824 x 5120 18.2 us with two, 20.6 with one).
+template <class E, int B, class S>
+__device__ __forceinline__ uint32_t xitem_dwords(uint32_t nch, const S& st) {
+    return kM4<B> || wide_chunks(E::ENC) ? st.b * xrow_dwords<E, B>(nch) + st.u * XTile<E>::XPW
+                                         : st.item * XTile<E>::XPW;
+}
 template <class E, int B>
 __device__ __forceinline__ const float* xconsts(const uint8_t* lds, uint32_t nch) {
     return reinterpret_cast<const float*>(lds) + (size_t)B * xrow_dwords<E, B>(nch);
 }
-// Stores (-C, s, s·Σx) of (row b, chunk u, group g).
-template <class E, int B>
-__device__ __forceinline__ void store_consts(uint8_t* lds, uint32_t nch, uint32_t b, uint32_t u, uint32_t g, float negc,
-                                             float s, float sm) {
+// Stores (-C, s, s·Σx) of group g of the staged chunk st (row b, chunk u, item = b·nch + u).
+template <class E, int B, class S>
+__device__ __forceinline__ void store_consts(uint8_t* lds, uint32_t nch, const S& st, uint32_t g, float negc, float s,
+                                             float sm) {
     using XT = XTile<E>;
     float* xc = const_cast<float*>(xconsts<E, B>(lds, nch));
     if constexpr (kM4<B>) {
-        float* c = xc + (size_t)(u * E::NG + g) * (XT::NCF * B) + b;
+        float* c = xc + (size_t)(st.u * E::NG + g) * (XT::NCF * B) + st.b;
         c[0] = negc;
         c[B] = s;
         if constexpr (XT::NCF == 4) c[2 * B] = sm;
     } else {
-        float* c = xc + ((size_t)(b * nch + u) * E::NG + g) * XT::NCF;
+        const uint32_t item = wide_chunks(E::ENC) ? st.b * nch + st.u : st.item;
+        float* c = xc + ((size_t)item * E::NG + g) * XT::NCF;
         if constexpr (XT::NCF == 4) *reinterpret_cast<float4*>(c) = make_float4(negc, s, sm, 0.0f);
         else *reinterpret_cast<float2*>(c) = make_float2(negc, s);
     }
@@ -191,7 +201,7 @@ struct GStage {
     static constexpr int TT = E::NT / SP;                   // code dwords per thread
     static constexpr int RPG = E::NG == 1 ? E::NXR : 1;     // runs of 4 per code dword in one group
     float v[TT][RPG][4];
-    uint32_t b, u;  // activation row, chunk
+    uint32_t b, u, item;  // activation row, chunk, b·nch + u
     uint32_t g;     // scale group within the chunk
     uint32_t q;     // part of the group (code dwords q·TT ..)
     bool live;      // the group exists: the thread stores
@@ -212,6 +222,7 @@ __device__ __forceinline__ void gstage_load(const GemvParams& p, uint32_t nch, u
     const uint32_t b = B == 1 ? 0u : item / nch, u = item - b * nch;
     s.b = b;
     s.u = u;
+    s.item = item;
     // Rows past the batch restage row 0: in bounds, and their sums are never
     // stored.  Activation offsets are 32-bit (the activations are < 4 GiB).
     const uint32_t base = (b < p.batch ? b : 0u) * p.ldx + E::xbase(u) + (uint32_t)E::RUNSTRIDE * s.g +
@@ -273,8 +284,7 @@ __device__ __forceinline__ void gstage_store(uint8_t* lds, uint32_t nch, const G
     float St = 0.0f;
     if constexpr (XT::NCF == 4) St = __uint_as_float(sp_reduce<SP>(__float_as_uint(Sx[0] + Sx[1]), fadd));
     if (s.live) {
-        uint32_t* xp = reinterpret_cast<uint32_t*>(lds) + s.b * xrow_dwords<E, B>(nch) + s.u * XT::XPW +
-                       s.q * (uint32_t)(S::TT * E::PPT);
+        uint32_t* xp = reinterpret_cast<uint32_t*>(lds) + xitem_dwords<E, B>(nch, s) + s.q * (uint32_t)(S::TT * E::PPT);
         if constexpr (E::NG == 1 && (S::TT * E::PPT) % 4 == 0) {
             // the thread's pairs are TT·PPT consecutive dwords
 #pragma unroll
@@ -294,7 +304,7 @@ __device__ __forceinline__ void gstage_store(uint8_t* lds, uint32_t nch, const G
         }
         if (s.q == 0) {
             const float sc = ldexpf(1.0f, ex - 14);
-            store_consts<E, B>(lds, nch, s.b, s.u, s.g, -Ct, sc, sc * St);
+            store_consts<E, B>(lds, nch, s, s.g, -Ct, sc, sc * St);
         }
     }
 }
@@ -339,8 +349,8 @@ __device__ __forceinline__ void stage_x_sp(uint8_t* lds, const GemvParams& p, MI
 template <class E>
 struct XStage {
     float v[E::NXR][4];
-    uint32_t b, u;  // activation row, chunk
-    bool live;      // the thread stores
+    uint32_t b, u, item;  // activation row, chunk, b·nch + u
+    bool live;            // the thread stores
 };
 
 // Issues the loads of staging thread idx (no use of the loaded values, so
@@ -354,6 +364,7 @@ __device__ __forceinline__ void xstage_load(const GemvParams& p, uint32_t nch, u
     const uint32_t b = B == 1 ? 0u : item / nch, u = item - b * nch;
     s.b = b;
     s.u = u;
+    s.item = item;
     // Rows past the batch restage row 0: in bounds, and their sums are never
     // stored.  Activation offsets are 32-bit (the activations are < 4 GiB).
     const uint32_t base = (b < p.batch ? b : 0u) * p.ldx + E::xbase(u) + (uint32_t)E::TSTRIDE * t;
@@ -426,7 +437,7 @@ __device__ __forceinline__ void xstage_store(uint8_t* lds, uint32_t nch, uint32_
         if constexpr (XT::NCF == 4) S[g] = __uint_as_float(lanes_reduce<E::NT>(__float_as_uint(S[g]), fadd));
     }
     if (s.live) {
-        uint32_t* dst = xp + s.b * xrow_dwords<E, B>(nch) + s.u * XT::XPW + t * (uint32_t)E::PPT;
+        uint32_t* dst = xp + xitem_dwords<E, B>(nch, s) + t * (uint32_t)E::PPT;
         if constexpr (E::PPT % 4 == 0) {
 #pragma unroll
             for (int h = 0; h < E::PPT; h += 4)
@@ -439,7 +450,7 @@ __device__ __forceinline__ void xstage_store(uint8_t* lds, uint32_t nch, uint32_
 #pragma unroll
             for (int g = 0; g < E::NG; g++) {
                 const float sc = ldexpf(1.0f, ex[g] - 14);
-                store_consts<E, B>(lds, nch, s.b, s.u, (uint32_t)g, -C[g], sc, sc * S[g]);
+                store_consts<E, B>(lds, nch, s, (uint32_t)g, -C[g], sc, sc * S[g]);
             }
         }
     }
