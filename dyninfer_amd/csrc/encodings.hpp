@@ -62,6 +62,12 @@ __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t m, uint32_t b) {
     asm("" : "+v"(b));
     return (a & m) | b;
 }
+// The same as the written instruction: only for operands of v_dot2.
+__device__ __forceinline__ uint32_t and_or_asm(uint32_t a, uint32_t m, uint32_t b) {
+    uint32_t r;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(m), "v"(b));
+    return r;
+}
 
 // Selector for v_perm_b32 that extracts the dword starting `sh` bytes into a
 // 4-byte-aligned pair {hi, lo}, plus a fixed byte offset `add` (0 or 2).
@@ -72,12 +78,14 @@ __device__ __forceinline__ uint32_t realign_sel(uint32_t sh, uint32_t add) {
 // The four decoded pairs of a dword of nibble codes whose weights are
 // (i, i+2) [bits 0-3 and 16-19], (j, j+2) x16 [bits 4-7 and 20-23],
 // and the same one byte up [bits 8-11/24-27, 12-15/28-31].
+template <bool ASM = false>
 __device__ __forceinline__ void nibble_pairs(uint32_t d, uint32_t (&p)[4]) {
     const uint32_t d8 = d >> 8;
-    p[0] = and_or(d, 0x000F000Fu, kMagic);
-    p[1] = and_or(d, 0x00F000F0u, kMagic);
-    p[2] = and_or(d8, 0x000F000Fu, kMagic);
-    p[3] = and_or(d8, 0x00F000F0u, kMagic);
+    auto f = [](uint32_t a, uint32_t m) { return ASM ? and_or_asm(a, m, kMagic) : and_or(a, m, kMagic); };
+    p[0] = f(d, 0x000F000Fu);
+    p[1] = f(d, 0x00F000F0u);
+    p[2] = f(d8, 0x000F000Fu);
+    p[3] = f(d8, 0x00F000F0u);
 }
 
 // Raw dwords of a 2-byte-aligned GGUF block: NDW dwords from the 4-byte-

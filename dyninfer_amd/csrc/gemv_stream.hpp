@@ -149,7 +149,10 @@ __device__ __forceinline__ float stream_chunk(const typename E::Chunk& c, const 
 #pragma unroll
     for (int t = 0; t < E::NT; t++) {
         uint32_t pr[E::PPT], xv[E::PPT];
-        E::pairs(c, t, pr);
+        // (Q4_K's loop comes out better around the written instruction: 24576 x 4096 13.7 ->
+        // 13.1 us, 151936 x 1024 19.4 -> 18.4; Q4_0's and Q5_K's do not, nor Q4_K's pipeline)
+        if constexpr (E::ENC == ENC_Q4_K) nibble_pairs<true>(c.q[t], pr);
+        else E::pairs(c, t, pr);
         load_xpairs<E>(xq, t, xv);
 #pragma unroll
         for (int h = 0; h < E::PPT; h++) {
