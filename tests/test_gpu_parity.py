@@ -140,14 +140,13 @@ LATENCY8_CASES += [(g, 6150, 1056) for g in (oracle.Q4_0, oracle.Q8_0)]
 @pytest.mark.parametrize("gtype,n,k", LATENCY8_CASES, ids=[f"{oracle.NAMES[g]}-{n}x{k}" for g, n, k in LATENCY8_CASES])
 @pytest.mark.parametrize("batch,xbf16", [(3, True), (4, False), (6, False), (8, False), (8, True)])
 def test_gemv_latency_mode_eight_rows(ctx, gtype, n, k, batch, xbf16):
-    """3-8 activation rows on small launches.  At 5-8 rows latency mode (one
-    wave per row block with all of a lane's chunks loaded at once) at 1 chunk
-    per lane (K = 2048) or 2 (K = 3072, where the lanes past the last chunk add
-    zero, 4096, and 1056 in 32 lanes); at 3-4 rows latency mode at 1 chunk,
-    the persistent pipeline at 2.  The 8-row kernel of 2 chunks is built for
-    256-thread workgroups and must never be launched with 512, including at
-    6150 rows, where 256 and 512 threads put the same number of waves on the
-    busiest CU."""
+    """3-8 activation rows on small launches, in latency mode (all of a lane's
+    chunks loaded at once; a row block is four rows by sixteen lanes).  Up to
+    1024 rows four waves share a row block, with 1 chunk per lane (K = 2048) or
+    2 (K = 3072, where the lanes past the last chunk add zero, and 4096); 6150
+    rows (1538 row blocks) of K = 1056 have one wave each, 3 chunks per lane in
+    the kernels of 4, where 256 and 512 threads put the same number of waves on
+    the busiest CU."""
     w, data = gguf(gtype, n, k, seed=500 + n + batch)
     x = oracle.randn(batch * k, seed=n + batch).reshape(batch, k)
     if xbf16:
@@ -173,40 +172,49 @@ def test_gemv_multi_qkv(ctx, batch):
         assert err <= XF16, err
 
 
-# 5..16 activation rows on at least 384 tiles of 16 weight rows (K a
-# multiple of 256) take the MFMA GEMV (every weight decoded once for all
-# rows): ragged rows, task counts needing padding tasks (Q4_0 1280 = 5 tasks
-# of 8 blocks, Q6_K 2304 = 9 super-blocks, rows alternating 4- and 2-byte
-# alignment), K split over LDS segments (12288: three launches, the later
-# ones adding with atomics), bf16 outputs, a weight base 2 bytes past a
-# 4-byte boundary; K = 1056 (not whole tasks) stays on the VALU GEMV.
+# The 16-row MFMA GEMV (every weight decoded once for all rows; K a multiple of
+# 256): 9..16 activation rows, 5..8 from 8 MB or 1024 tiles of 16 weight rows,
+# 3..4 of Q6_K from 4096 tiles.  Ragged rows, task counts needing padding tasks
+# (Q4_0 1280 = 5 tasks of 8 blocks, Q6_K 2304 = 9 super-blocks, rows alternating
+# 4- and 2-byte alignment), K split over LDS segments (12288: three launches,
+# the later ones adding with atomics), bf16 outputs, a weight base 2 bytes past
+# a 4-byte boundary.  test_decode_route_cover.py holds the lists to these routes.
 MFMA_CASES = [
-    (oracle.Q4_0, 6144, 1024, 5, False, 0), (oracle.Q4_0, 6144, 1024, 16, False, 0),
-    (oracle.Q4_0, 6150, 1280, 9, False, 2), (oracle.Q4_0, 6150, 1056, 9, False, 2),
+    (oracle.Q4_0, 6144, 1024, 16, False, 0), (oracle.Q4_0, 6150, 1280, 9, False, 2),
     (oracle.Q4_0, 6144, 4096, 16, True, 0),
     (oracle.Q4_0, 6144, 12288, 7, False, 0), (oracle.Q4_0, 8000, 2048, 12, True, 0),
-    (oracle.Q6_K, 6144, 1024, 5, False, 0), (oracle.Q6_K, 6144, 4096, 16, True, 0),
+    (oracle.Q6_K, 6144, 4096, 16, True, 0),
     (oracle.Q6_K, 6150, 2304, 9, False, 2), (oracle.Q6_K, 6144, 12288, 7, False, 0),
     (oracle.Q6_K, 8000, 4096, 12, True, 2),
     # whole tiles per wave (>= 1024 tiles) and few tiles shared by a workgroup's waves
     (oracle.Q4_0, 20480, 1024, 9, False, 0), (oracle.Q6_K, 17000, 1024, 16, True, 2),
     (oracle.Q6_K, 1040, 4096, 16, False, 0), (oracle.Q6_K, 4096, 12288, 16, False, 0),
     (oracle.Q4_0, 4096, 4096, 8, True, 0),
-    # 3-4 rows: launches of >= 1024 tiles, and Q4_0 from 384 tiles (split mode)
-    (oracle.Q6_K, 17000, 1024, 4, False, 0), (oracle.Q4_0, 20480, 1024, 3, True, 2),
-    (oracle.Q4_0, 6144, 4096, 4, False, 0), (oracle.Q4_0, 6150, 4096, 3, True, 2),
-    # more rows than one VALU register pass: whole tiles from 128 tiles
-    (oracle.Q4_0, 2048, 1024, 12, False, 0), (oracle.Q6_K, 2570, 1024, 8, True, 2),
+    # whole tiles from 128 tiles
+    (oracle.Q4_0, 2048, 1024, 12, False, 0),
     # split mode, more tiles than resident workgroups: two 4-wave tile groups per
     # workgroup (an odd tile count leaves one group a recomputed, unstored tile)
     (oracle.Q4_0, 6160, 1024, 16, False, 0), (oracle.Q6_K, 6160, 1024, 16, True, 2),
     (oracle.Q4_0, 4104, 2048, 16, True, 0),
+    # 3-4 rows, ragged
+    (oracle.Q6_K, 65530, 512, 3, False, 0), (oracle.Q6_K, 65540, 256, 4, True, 2),
+    # 5-8 rows: 1025 tiles, and 8 MB
+    (oracle.Q4_0, 16390, 512, 5, False, 0), (oracle.Q6_K, 16390, 512, 8, True, 2),
+    (oracle.Q6_K, 6150, 2048, 6, False, 2),
+]
+# Beside its lines: K = 1056 is not whole tasks, and fewer rows on smaller launches run on
+# the register batches (4x4 MFMAs, each weight decoded once a pass).
+MFMA_NOT_CASES = [
+    (oracle.Q4_0, 6150, 1056, 9, False, 2), (oracle.Q4_0, 6144, 1024, 5, False, 0),
+    (oracle.Q6_K, 6144, 1024, 5, False, 0), (oracle.Q6_K, 2570, 1024, 8, True, 2),
+    (oracle.Q6_K, 17000, 1024, 4, False, 0), (oracle.Q4_0, 20480, 1024, 3, True, 2),
+    (oracle.Q4_0, 6144, 4096, 4, False, 0), (oracle.Q4_0, 6150, 4096, 3, True, 2),
 ]
 
 
-@pytest.mark.parametrize("gtype,n,k,batch,ybf16,off", MFMA_CASES,
+@pytest.mark.parametrize("gtype,n,k,batch,ybf16,off", MFMA_CASES + MFMA_NOT_CASES,
                          ids=[f"{oracle.NAMES[c[0]]}-{c[1]}x{c[2]}-b{c[3]}{'-bf16' if c[4] else ''}{'-off2' if c[5] else ''}"
-                              for c in MFMA_CASES])
+                              for c in MFMA_CASES + MFMA_NOT_CASES])
 def test_gemv_mfma(ctx, gtype, n, k, batch, ybf16, off):
     w, data = gguf(gtype, n, k, seed=n + k + batch, off=off)
     x = oracle.randn(batch * k, seed=batch).reshape(batch, k)
@@ -231,8 +239,8 @@ def test_gemv_mfma(ctx, gtype, n, k, batch, ybf16, off):
 # are identical (K segments add atomically, in either order: within 1e-6 of
 # Σ|w||x|).  The workspace starts as 0xFF bytes (NaN in f16 and f32), so
 # activation rows the prep kernel leaves unstaged (past the batch rounded up
-# to 4, 8 or 16) must not reach a stored output.  5..8 rows take the MFMA GEMV
-# from 8 MB or 1024 tiles: 1025 tiles, the oracle on the first 2048 rows.
+# to 4, 8 or 16) must not reach a stored output.  The oracle checks the first
+# 2048 rows.
 PRESTAGE_CASES = [c for c in MFMA_CASES if c[2] >= 2048 and (c[3] > 8 or c[2] > 4096)] + [
     (oracle.Q4_0, 16400, 8192, 5, False, 0), (oracle.Q4_K, 6144, 4096, 16, False, 0),
     # 3..8 rows whose activation tile is too long for the 4x4 kernels' one pass
@@ -447,10 +455,12 @@ def test_gemv_mfma_grouped(ctx, gtype):
 
 @pytest.mark.parametrize("gtype", [oracle.Q4_0, oracle.Q6_K], ids=oracle.NAMES.get)
 @pytest.mark.parametrize("lo,hi", [(6, 8), (-30, -28), (-8, 8)])
-def test_gemv_mfma_activation_range(ctx, gtype, lo, hi):
+@pytest.mark.parametrize("batch", [8, 9])
+def test_gemv_mfma_activation_range(ctx, gtype, lo, hi, batch):
     """The MFMA path's per-(row, task) power-of-two scaling over magnitudes f16
-    cannot hold unscaled, mixed within a task, and a zero run."""
-    n, k, batch = 6144, 2048, 8
+    cannot hold unscaled, mixed within a task, and a zero run (at 8 rows Q4_0,
+    below 8 MB, runs on the register batches: scaled per 32 weights)."""
+    n, k = 6144, 2048
     w, data = gguf(gtype, n, k, seed=17 + gtype)
     x = _ranged_x(batch, k, seed=(lo + 100) * 7 + (hi + 100), lo=lo, hi=hi)
     y = ctx.qlinear(w, dev(x)).cpu().numpy()
@@ -479,24 +489,24 @@ def test_gemv_mlx_bf16_io(ctx, sdtype, n, k, g, batch):
     assert np.all(err <= TOL + rounding), err.max()
 
 
-# MLX affine U4 on the MFMA GEMV (more than 8 rows, or 3-4 on >= 1024 tiles;
-# K a multiple of 256):
-# whole tiles per wave (>= 1024 tiles, or >= 384 with fewer than 8 tasks),
-# split mode, group sizes 32 / 64 / 128, every scale dtype, bf16 and f32
-# activations.
+# MLX affine U4 on the MFMA GEMV (9..16 rows, 5..8 from 8 MB or 1024 tiles; K a
+# multiple of 256): whole tiles per wave (>= 1024 tiles, or >= 384 with fewer
+# than 8 tasks), split mode, group sizes 32 / 64 / 128, every scale dtype, bf16
+# and f32 activations.
 MLX_MFMA_CASES = [
     (6144, 1024, 64, oracle.D_BF16, 16, True), (20000, 1024, 64, oracle.D_F16, 12, True),
     (1024, 3072, 64, oracle.D_F16, 12, True), (3072, 2048, 32, oracle.D_F32, 16, True),
     (2048, 4096, 128, oracle.D_BF16, 9, False), (4100, 2048, 64, oracle.D_BF16, 9, False),
-    (20000, 1024, 64, oracle.D_BF16, 4, True),
-    (4096, 1024, 64, oracle.D_BF16, 16, True),  # 256 tiles, split (two VALU passes at 16 rows)
+    (20000, 512, 64, oracle.D_BF16, 5, True), (16400, 256, 32, oracle.D_F32, 8, False),
+    (4096, 1024, 64, oracle.D_BF16, 16, True),  # 256 tiles, split
     (6160, 1024, 64, oracle.D_BF16, 16, True),  # 385 tiles: two 4-wave tile groups per workgroup
 ]
+MLX_MFMA_NOT_CASES = [(20000, 1024, 64, oracle.D_BF16, 4, True)]  # 3..4 rows: the register batches
 
 
-@pytest.mark.parametrize("n,k,g,sdtype,batch,xbf16", MLX_MFMA_CASES,
+@pytest.mark.parametrize("n,k,g,sdtype,batch,xbf16", MLX_MFMA_CASES + MLX_MFMA_NOT_CASES,
                          ids=[f"{c[0]}x{c[1]}-g{c[2]}-s{c[3]}-b{c[4]}{'-bf16io' if c[5] else '-f32io'}"
-                              for c in MLX_MFMA_CASES])
+                              for c in MLX_MFMA_CASES + MLX_MFMA_NOT_CASES])
 def test_gemv_mfma_mlx(ctx, n, k, g, sdtype, batch, xbf16):
     packed, sc, bi = oracle.synth_mlx_u4(n, k, g, sdtype, seed=n + k + g + batch)
     w = d.QWeight(d.ENC_MLX_U4, n, k, dev(packed), dev(sc), dev(bi), g, sdtype)
@@ -531,32 +541,30 @@ def test_gemv_mlx_f32_io(ctx, batch, k):
 
 
 # ----------------------------------------------------------------- GEMM (MFMA prefill)
-# Shapes that select every launch plan the GEMM's planner picks for Q4_0, Q4_1
-# and Q8_0: TM = 2 or 4 activation row blocks and NB = 2 or 3 weight row
-# blocks (of 32) per wave, S = 1, 2 or 4 K slices per 4-wave workgroup; plus
-# ragged rows and columns, one-chunk K, and chunk counts no split divides.
-# (m, n, k) -> (TM, NB, S) for Q4_0:
+# Model shapes and the edges of the GEMM: ragged rows and columns, one-chunk K,
+# chunk counts no K split divides.  (The shapes of test_gpu_gemm_plans.py reach
+# every configuration of the planner.)
 GEMM_SHAPES = [(17, 130, 64),      # one 64-k chunk: Q4_1/Q8_0 GEMM (Q4_0 takes 16-row GEMV chunks)
-               (40, 256, 64),      # one chunk, every type on the GEMM (2, 2, 1)
+               (40, 256, 64),      # one chunk, every type on the GEMM
                (64, 1000, 64),     # one chunk, ragged N
-               (17, 256, 1024),    # (2, 2, 4)
-               (20, 20000, 256),   # (2, 3, 2)
-               (33, 512, 2048),    # (2, 2, 4)
-               (50, 20000, 256),   # (2, 3, 2)
-               (100, 300, 128),    # (2, 2, 2), two-chunk slices
+               (17, 256, 1024),
+               (20, 20000, 256),
+               (33, 512, 2048),
+               (50, 20000, 256),
+               (100, 300, 128),    # two chunks
                (200, 384, 1024),   # ragged last row tile
-               (512, 3072, 1024),  # (2, 3, 4) (Qwen3-0.6B gate/up)
-               (512, 1024, 3072),  # (2, 2, 4) (down)
+               (512, 3072, 1024),  # Qwen3-0.6B gate/up
+               (512, 1024, 3072),  # down
                (512, 6144, 1024),
-               (768, 2048, 1024),  # (4, 2, 4)
-               (768, 3072, 1024),  # (2, 3, 2)
-               (1536, 2048, 1024),  # (4, 2, 2)
-               (2048, 3072, 1024),  # (4, 2, 1)
+               (768, 2048, 1024),
+               (768, 3072, 1024),
+               (1536, 2048, 1024),
+               (2048, 3072, 1024),
                (2000, 3000, 1024),  # ragged rows and columns
                (2048, 64, 8128),   # 127 chunks of 64 k: no K split divides them
                (300, 200, 4032),   # 63 chunks
-               (48, 256, 12288),   # activation staging: 24 register slots per lane
-               (40, 128, 16384)]   # activation staging: second pass reloads the row
+               (48, 256, 12288),   # activation staging: long rows
+               (40, 128, 16384)]   # activation staging: longer rows
 GEMM_TYPES = [oracle.Q4_0, oracle.Q4_1, oracle.Q8_0]
 
 
@@ -582,17 +590,17 @@ def test_gemm(ctx, gtype, m, n, k, ybf16):
     assert np.all(err <= 2.0 ** -11 + 1e-5 + extra), err.max()
 
 
-# Q6_K: K a multiple of 256, the GEMM from 33 rows (shape -> TM, NB, S)
+# Q6_K: K a multiple of 256, the GEMM from 33 rows
 GEMM_SHAPES_Q6K = [(50, 20000, 256),
                    (64, 1000, 512),
                    (100, 300, 512),
                    (200, 384, 1024),
-                   (512, 3072, 1024),  # (2, 3, 4)
-                   (512, 1024, 3072),  # (2, 2, 4)
+                   (512, 3072, 1024),
+                   (512, 1024, 3072),
                    (512, 6144, 1024),
-                   (768, 2048, 1024),  # (2, 2, 2)
-                   (768, 3072, 1024),  # (4, 2, 2)
-                   (2048, 3072, 1024),  # (4, 2, 1)
+                   (768, 2048, 1024),
+                   (768, 3072, 1024),
+                   (2048, 3072, 1024),
                    (2000, 3000, 1024),  # ragged
                    (300, 200, 4096)]
 

@@ -120,8 +120,7 @@ def test_prefill_multi(ctx, kind, rows):
 @pytest.mark.parametrize("ybf16", [False, True], ids=["yf32", "ybf16"])
 def test_gemm_q4_0_f32_activations(ctx, m, n, k, ybf16):
     """The Q4_0 GEMM with f32 activations (the candidates' advertised input
-    type): each kernel path (K-split at M=128, 128x64 and 128x128 tiles),
-    ragged tiles."""
+    type): tiles and K splits of several sizes, ragged tiles."""
     w, wf = make(oracle.Q4_0, n, k, seed=m + n)
     xd, x = xs(m, k, seed=m * 3 + k, bf16=False)
     y = ctx.qlinear(w, xd, y_dtype=torch.bfloat16 if ybf16 else torch.float32)
