@@ -210,17 +210,16 @@ size_t esize(uint32_t dt) { return dt == DYNINFER_DTYPE_F32 ? 4 : 2; }
 // Whether `rows` activation rows run the prefill GEMM (else the GEMV kernels
 // over 16-row chunks).  Q4_1, Q8_0 and MLX U4 take the GEMM from 17 rows (MLX
 // 4096x1024: 13.4 against 17.0 us at 17 rows, 19.8 against 380 us at 512).
-// The 16-row GEMV of Q4_0, Q6_K and Q4_K runs on MFMA, and two of its chunks
-// (17..32 rows) mostly take less time than staging plus a GEMM with so few
-// workgroups (Q4_0 4096x4096 at 24 rows: 21.5 against 23.8 us; Q6_K 1024x4096
-// 23.2 against 35.6 us), three never do (40 rows: Q4_0 4096x4096 32.2 against
-// 24.6 us, 12288x4096 52.4 against 28.2 us); with K above 8192 the MFMA GEMV
-// splits K over launches and the GEMM wins from 17 rows (Q4_0 4096x12288:
-// 60.9 against 73.2 us, Q4_K 66.9 against 81.8 us).  Except Q6_K with f32
-// outputs: at K above 8192 its GEMM has few row tiles, each decoding long
-// Q6_K slices, and the 16-row MFMA GEMV chunks win up to 32 rows (4096x12288:
-// 46 against 102 us at 17 rows, 71 against 103 at 32; 107 against 106 at 48).
-// With bf16 outputs the MFMA GEMV does not split K, so the GEMM stays.
+// The encodings whose 16-row GEMV runs on MFMA take two of its chunks at 17..32 rows
+// of K up to 8192, Q6_K with f32 outputs of any K; above K = 8192, where the MFMA GEMV
+// splits K over launches (bf16 outputs: not at all), the GEMM.  Per call on rotating
+// weights, f32 activations, chunks against the GEMM: Q6_K 4096 x 4096 17 rows 15.2 us,
+// 19.2, 32 rows 18.7, 19.1, 24576 x 4096 24 rows 52.2, 58.4, 4096 x 12288 38.8, 46.8.
+// For the rest the line dates from a slower GEMM: near 17 rows the two are level
+// (Q4_0 4096 x 4096 12.1, 11.5, 12288 x 4096 21.7, 22.4, 2048 x 8192 14.8, 17.5), from
+// 20 the GEMM is ahead (24 rows: Q4_0 4096 x 4096 16.4, 11.3, 24576 x 4096 42.5, 28.2,
+// Q4_K 46.7, 31.2, Q5_K 56.8, 36.9, IQ4_XS 55.9, 33.8), as in Q6_K up to K = 1024
+// (6144 x 1024 13.1, 8.2).
 bool has_prefill_gemm(uint32_t enc, uint32_t N, uint32_t K, uint32_t rows, bool y_bf16) {
     const bool mfma_gemv = enc == DYNINFER_ENC_GGUF_Q4_0 || enc == DYNINFER_ENC_GGUF_Q6_K ||
                            enc == DYNINFER_ENC_GGUF_Q4_K || enc == DYNINFER_ENC_GGUF_Q5_K ||

@@ -29,11 +29,12 @@
 //     NB = 1 over shared fragments is bound by LDS (1 KiB per MFMA, 128 B/clk); small
 //     M and short K are bound by the first copies' latency and the epilogue, so
 //     those take many small tiles with K split over the waves (gemm_plan).
-//     Measured (against the same tile shapes with a two-slot ring shared by four
-//     waves, one launch per weight): Q4_0 2048 x 24576 x 4096 508 -> 362 us (1.14
-//     PFLOP/s; a library f16 GEMM of the shape 326), Q6_K 2048 x 4096 x 12288 468 ->
-//     255, 512 x 4096 x 12288 204 -> 88, Q5_K 45 x 24576 x 4096 54 -> 31, Q4_0
-//     512 x 4096 x 1024 in three weights 27 -> 9.5 us.
+//     Measured (kernel trace, median and least of the launches in a stream of calls,
+//     against the same tile shapes with a two-slot ring shared by four waves, one
+//     launch per weight): Q4_0 2048 x 24576 x 4096 507 (464 at least) -> 405 us (352,
+//     1.17 PFLOP/s), Q6_K 2048 x 4096 x 12288 417 (410) -> 290 (277), 512 x 4096 x
+//     12288 189 (186) -> 103 (101), Q5_K 45 x 24576 x 4096 51.3 (50.0) -> 35.3 (34.7),
+//     Q4_0 512 x 4096 x 1024 in three weights 23.4 (22.4) -> 10.9 (10.8).
 //   * Every lane decodes 32 weights of one row per N-block straight into A
 //     operands: lane l takes weight row l % 32 of a 32-row block and its half
 //     h = l / 32 of the chunk (the block h, for blocks of 32), so an MFMA k step

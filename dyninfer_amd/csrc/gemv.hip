@@ -141,7 +141,7 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
     hipError_t le = lds_limit(&lim);
     if (le != hipSuccess) return le;
     uint32_t B = 1;
-    while (B < batch && B < max_register_batch(enc)) B *= 2;
+    while (B < batch && B < kMaxRegisterBatch) B *= 2;
     while (B > 1 && xtile_bytes(enc, B, K) > lim) B /= 2;
     if (xtile_bytes(enc, B, K) > lim) return hipErrorInvalidValue;
     if (batch > B) {

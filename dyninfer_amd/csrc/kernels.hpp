@@ -75,7 +75,7 @@ __host__ __device__ constexpr uint64_t xtile_bytes(uint32_t enc, uint32_t B, uin
 }
 // Widest activation batch one GEMV launch holds in registers (wider batches
 // run as several launches).
-__host__ __device__ constexpr uint32_t max_register_batch(uint32_t) { return 8u; }
+constexpr uint32_t kMaxRegisterBatch = 8;
 // Latency mode with four waves per row block (with the chunks per lane in the low bits).
 // kOneshotWide: four row blocks to a workgroup (64-weight chunks: of two waves each);
 // kOneshotThree: three.
@@ -168,9 +168,9 @@ inline uint64_t prefill_workspace_bytes(uint32_t M, uint32_t K) {
     return prefill_xh_bytes(M, K) + (((uint64_t)M + 255u) & ~(uint64_t)255u) * 4u;
 }
 
-// Prefill GEMM launch plan (gemm.hip): workgroups of s·wn waves, each owning a
-// (32·tm) x (32·nb·wn) tile of one weight's Y, the waves split over s K slices
-// and wn column subtiles.
+// Prefill GEMM launch plan (gemm.hip): workgroups of s·wn·wm waves, each owning a
+// (32·tm·wm) x (32·nb·wn) tile of one weight's Y, the waves split over s K slices,
+// wn column and wm row subtiles.
 struct GemmPlan {
     uint32_t tm, nb, s, wn, wm;
     uint32_t mt, nt;  // workgroup tiles along M and (every weight's) along N

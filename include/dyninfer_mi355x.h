@@ -128,15 +128,15 @@ const char* dyninfer_mi355x_last_error(void);
  * gguf_codegen.rs:157-159).  `rows` = activation rows (1..16 for decode; any for prefill).
  * x: [rows, K] row-major, 16-byte aligned, dtype x_dtype (f32 or bf16, every encoding);
  * y: [rows, N], dtype y_dtype (f32 or bf16).
- *   rows <= 16: the decode GEMV kernels (3..8 rows on 4x4 MFMAs; 5..16 rows of large
- *     Q4_0, Q6_K, Q4_K, Q5_K, IQ4_XS and MLX weights, and the largest Q6_K from 3, on
- *     16-row MFMAs), activations rounded to f16 after a power-of-two scaling per scale
- *     group;
+ *   rows <= 16: the decode GEMV kernels, activations rounded to f16 after a power-of-two
+ *     scaling per scale group: 1..2 rows on the vector units, 3..8 on 4x4 MFMAs, 9..16 of
+ *     Q4_0, Q6_K, Q4_K, Q5_K, IQ4_XS and MLX weights on 16-row MFMAs, and fewer where
+ *     those are the faster ones (5..8 of large weights, 3..4 of the largest Q6_K and of
+ *     large weights whose K is too long for one pass);
  *   rows >= 17: the prefill path.  Q4_1, Q8_0 and MLX U4 from 17 rows, Q4_0, Q6_K and
  *     the K-quants / IQ4_XS from 33 rows, or from 17 when K > 8192 except Q6_K with f32
- *     outputs (below that two 16-row MFMA GEMV chunks are mostly faster), K a multiple
- *     of 64 (256 for the super-block
- *     encodings): x is staged once per call as f16 MFMA operand fragments,
+ *     outputs (below that two 16-row MFMA GEMV chunks), K a multiple of 64 (256 for the
+ *     super-block encodings): x is staged once per call as f16 MFMA operand fragments,
  *     each row scaled by a power of two (RNE) and the rows padded with zeros to a
  *     multiple of 32, into the caller's workspace; then one MFMA GEMM launch
  *     decodes the GGUF blocks or MLX words straight into MFMA operands.  Every other
