@@ -1133,6 +1133,26 @@ inline void split_waves(GemvParams& p, uint32_t rows_per_rb, uint32_t threads) {
     }
 }
 
+// Weight rows on the busiest CU of that grid, workgroup i running on CU i % cus: its
+// waves' first ones have one row block more than the rest, so one of the CUs where a
+// problem's waves begin.
+inline uint64_t busiest_cu_rows(const GemvParams& p, uint32_t rows_per_rb, uint32_t waves, uint32_t cus) {
+    uint64_t most = 0;
+    for (uint32_t k = 0; k < p.nprob; k++) {
+        uint64_t rbs = 0;
+        for (uint32_t wg = ((k ? p.wave_end[k - 1] : 0u) + waves - 1) / waves % cus; wg < p.grid; wg += cus)
+            for (uint32_t i = 0; i < p.nprob; i++) {
+                const uint32_t b = i ? p.wave_end[i - 1] : 0u, e = p.wave_end[i];
+                const uint32_t lo = wg * waves > b ? wg * waves : b, hi = (wg + 1) * waves < e ? (wg + 1) * waves : e;
+                if (lo >= hi) continue;
+                const uint32_t all = (p.n[i] + rows_per_rb - 1) / rows_per_rb, more = b + all % (e - b);
+                rbs += (uint64_t)(hi - lo) * (all / (e - b)) + (more > lo ? (more < hi ? more : hi) - lo : 0u);
+            }
+        most = rbs > most ? rbs : most;
+    }
+    return most * rows_per_rb;
+}
+
 typedef void (*GemvKernel)(GemvParams);
 constexpr int kGemvMaxTiles = 6;
 
@@ -1167,8 +1187,17 @@ struct GemvTile {
 // rule takes the first-listed workgroup size only: at one workgroup per CU
 // (the 8B Q6_K down_proj at 4 rows, 96 KiB of activations) 256 threads split
 // evenly with half the waves, 23.3 us per launch against 17.9.
+// cu_rows (4 and 8 activation rows, 32-weight chunks): row blocks of 4 or 8 rows
+// split coarsely, so ties in rows per wave go by the busiest CU's true rows
+// (busiest_cu_rows), 256 threads only where these are below 4/5 (each workgroup stages
+// the activations).  20000 rows, 8 a wave either way: in 2-row tiles 57 CUs have two
+// workgroups and the rest one, in 1-row tiles 113 have 24 row blocks and the rest 16
+// (us per launch at 4 rows: Q8_0 20000 x 7168 48.9 -> 35.1, IQ4_XS 18432 x 6144 32.4 ->
+// 24.9, Q4_0 24576 x 5120 21.4 -> 17.7; 8 rows: Q8_0 18432 x 3584 28.2 -> 22.8; but Q8_0
+// 18432 x 2048 13.1 -> 13.9).  MLX tiles came out 2% slower by it and 8% on 50000 x 5120,
+// 64-weight chunks, which have 1-row tiles only, from 0.84 to 1.09 of their time.
 inline hipError_t launch_persistent_best(const GemvTile* t, int n, const GemvParams& p0, size_t lds,
-                                         uint32_t cpl, hipStream_t st) {
+                                         uint32_t cpl, hipStream_t st, bool cu_rows = false) {
     const uint32_t groups = 64u >> p0.lanes_log2;  // lane groups per wave
     uint64_t total_rows = 0;
     for (uint32_t k = 0; k < p0.nprob; k++) total_rows += p0.n[k];
@@ -1196,12 +1225,14 @@ inline hipError_t launch_persistent_best(const GemvTile* t, int n, const GemvPar
             rbs = r > rbs ? r : rbs;
         }
         const uint64_t rows = rbs * rows_per_rb;
-        const uint64_t load = rows * waves * (((uint64_t)q.grid + (uint64_t)cus - 1) / (uint64_t)cus);
+        uint64_t load = rows * waves * (((uint64_t)q.grid + (uint64_t)cus - 1) / (uint64_t)cus);
         if (even < 0 && t[i].threads == t[0].threads && rbs * cpl >= 8 &&
             load * 100 <= total_rows * 105 / (uint64_t)cus) {
             even = i;
             chosen_even = q;
         }
+        if (cu_rows)
+            load = busiest_cu_rows(q, rows_per_rb, (uint32_t)waves, (uint32_t)cus) * (t[i].threads == 256u ? 5u : 4u);
         if (rows < best || (rows == best && load < best_load)) {
             best = rows;
             best_load = load;
@@ -1391,7 +1422,8 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
     }
 #undef DMX_CASE
     if (n == 0) return hipErrorInvalidValue;
-    return launch_persistent_best(t, n, p, lds, (nch + (1u << p.lanes_log2) - 1u) >> p.lanes_log2, st);
+    return launch_persistent_best(t, n, p, lds, (nch + (1u << p.lanes_log2) - 1u) >> p.lanes_log2, st,
+                                  B >= 4 && !wide_chunks(E::ENC));
 }
 
 

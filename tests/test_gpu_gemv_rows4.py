@@ -84,6 +84,7 @@ SHAPES = [
     (4, [8200], 7680),            # one workgroup to a CU, more row blocks than they take at once
     (8, [2100, 2200], 5120),      # the pipeline, one workgroup to a CU
     (4, [33001], 256),
+    (7, [16901], 2560),           # the pipeline, one row a lane group
     (8, [8197, 8197], 768),
     (16, [517], 1280),            # two passes, or the 16-row kernels
     (11, [4100], 1024),
