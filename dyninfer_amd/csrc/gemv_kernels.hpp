@@ -1376,6 +1376,7 @@ hipError_t launch_gguf_gemv_x(const GemvParams& p, uint32_t B, uint32_t oneshot,
             if constexpr (xtile_chunk_bytes(E::ENC) < 96u) DMX_ONESHOT_SPLIT(4, 8)
             DMX_ONESHOT_SPLIT(8, 3)
             DMX_ONESHOT_SPLIT(8, 4)
+            DMX_ONESHOT_FOUR_THREE(4, 3)
             DMX_ONESHOT_FOUR_THREE(4, 4)
             DMX_ONESHOT_FOUR_THREE(4, 5)
             DMX_ONESHOT_FOUR_THREE(4, 6)

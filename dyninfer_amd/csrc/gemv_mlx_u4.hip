@@ -47,6 +47,7 @@ hipError_t launch_mlx(const GemvParams& p, uint32_t B, uint32_t oneshot, hipStre
         DMX_ONESHOT_SPLIT(8, 2)
         DMX_ONESHOT_SPLIT(8, 3)
         DMX_ONESHOT_SPLIT(8, 4)
+        DMX_ONESHOT_FOUR_THREE(4, 3)
         DMX_ONESHOT_FOUR_THREE(4, 4)
         DMX_ONESHOT_FOUR_THREE(4, 5)
         DMX_ONESHOT_FOUR_THREE(4, 6)

@@ -67,7 +67,9 @@ SHAPES = [
     (3, [1027, 900], 512),        # a wave each, one chunk a lane
     (5, [997], 4352),             # eight rows, four waves per row block, three chunks a lane
     (7, [2047], 6656),            # ... four
-    (4, [2100], 8192),            # three row blocks to a workgroup, four chunks a lane
+    (4, [2500], 5120),            # three row blocks to a workgroup, three chunks a lane
+    (3, [3333], 4352),            # ... four
+    (4, [2100], 8192),            # three, four chunks a lane
     (3, [2501], 10240),           # ... five
     (4, [3070], 12288),           # ... six
     (4, [2053], 13312),           # ... seven
