@@ -213,9 +213,10 @@ hipError_t gemv_launch(uint32_t enc, const GemvProblem* probs, int nprob, uint32
         // 11.9, 9.8, 8.5, Q8_0 3072 x 10240 21.2, 15.8, 14.6, IQ4_XS 2500 x 12288 18.2, 16.5,
         // 13.6; the pipeline and three: MLX 2560 x 6144 11.9, 6.7, Q4_0 8.1, 6.2; and four: MLX
         // 4096 x 6144 14.2, 8.2, Q4_0 4096 x 12288 17.4, 13.6; at 8 rows Q8_0 3000 x 6144 18.6,
-        // 15.8, 14.6, but bf16 13.7, 16.2, 14.1, and at 4 rows 4096 x 7168 12.2, four 13.0).
+        // 15.8, 14.6, but bf16 13.7, 16.2, 14.1, and at 4 rows in four 4096 x 7168 12.2, 13.0,
+        // 4096 x 13312 20.0, 21.1, 3700 x 14336 21.2, 22.0).
         else if (!info.wide && room && rbs1 <= 1024u && cps >= 3u && cps <= (B == 4u ? 7u : 4u) &&
-                 !(enc == ENC_Q8_0 && x_bf16 && (B == 8u || (!one_per_cu && rbs1 > 768u))))
+                 !(enc == ENC_Q8_0 && x_bf16 && (B == 8u || rbs1 > 768u)))
             oneshot = (rbs1 <= 768u ? kOneshotThree : kOneshotWide) | cps;
         // 64-weight chunks at 4 rows, 513 to 1024 row blocks: the pipeline (four waves each
         // against it, two workgroups to a CU: Q4_K 3072 x 2560 8.0 -> 6.2, 3072 x 7168 15.8 ->

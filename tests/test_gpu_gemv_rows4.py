@@ -102,6 +102,6 @@ def test_shapes(kind):
 
 
 @pytest.mark.parametrize("kind", KINDS)
-@pytest.mark.parametrize("m,n,k", [(4, 1030, 2048), (5, 4099, 1024), (4, 2049, 12288)])
+@pytest.mark.parametrize("m,n,k", [(4, 1030, 2048), (5, 4099, 1024), (4, 2049, 12288), (4, 3077, 8192), (3, 2053, 5120)])
 def test_bf16(kind, m, n, k):
     check(d.Context(0), kind, m, [n], k, bf16=True)
